@@ -6,8 +6,8 @@
 // ... (G = grid size; `order` lists the matrices by decreasing n, so the
 // round-robin deal is a longest-first schedule).  Each matrix is factored in
 // place, right-looking over 16-column leaves:
-//   * wave 0 factors leaf p in registers (DPP row broadcasts), writes L_pp,
-//     accumulates log of the pivots and inverts L_pp into LDS;
+//   * wave 0 factors leaf p in registers (leaf_factor_invert), writes L_pp,
+//     accumulates log of the pivots and puts inv(L_pp) into LDS;
 //   * all waves form the panel L_Ip = A_Ip inv(L_pp)^T on the matrix cores
 //     (written to the matrix and kept in LDS);
 //   * all waves update the trailing lower tiles A_IJ -= L_Ip L_Jp^T with
@@ -63,29 +63,24 @@ struct View {
   }
 };
 
-// Wave 0: factor the leaf at g0 whose rows are in a[] (lane r + 16 q holds
-// row r), write L_pp to the matrix, accumulate log L_rr^2 of the valid rows
-// into logpart and put inv(L_pp) into Li; returns the failing pivot's column
-// (g0 + k) or -1.
+// Wave 0: factor the leaf at g0 held in f (row fragments), write L_pp to the
+// matrix, accumulate log L_rr^2 of the valid rows into logpart and put
+// inv(L_pp) into Li; returns the failing pivot's column (g0 + k) or -1.
 template <typename ST, bool LOWER>
-__device__ __forceinline__ int leaf_step(double (&a)[LEAF], const View<ST, LOWER> &v, int g0, double *Li,
+__device__ __forceinline__ int leaf_step(TileAcc<double> &f, const View<ST, LOWER> &v, int g0, double *Li,
                                          double &logpart) {
-  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-  double x[4], rpiv;
-  const int b = t16::leaf_factor_invert<double>(a, x, rpiv);
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  // the lane on the diagonal of X = inv(L_pp) holds 1 / L_rr
+  double rp = 1.0;
+  const int b = t16::leaf_factor_invert<double>(f, [&](int r, double, double x) {
+    Li[li * LL + lk + 4 * r] = x;
+    if (lk + 4 * r == li) rp = x;
+  });
   if (b >= 0) return g0 + b;
-  // log of this lane's own pivot L_rr^2 = -2 log(1 / L_rr), all rows at once
-  // (off the pivot chain); summed over the 16 rows once per matrix
-  if (q == 0 && g0 + r < v.n) logpart -= 2.0 * log(rpiv);
+  // log L_rr^2 = -2 log(1 / L_rr), summed over the leaf's rows once per matrix
+  if (lk == (li & 3) && g0 + li < v.n) logpart -= 2.0 * log(rp);
 #pragma unroll
-  for (int j = 0; j < 4; j++) {  // lane group q writes columns q + 4 j of its row
-    // a value select (a conditional over the array elements themselves
-    // would select their addresses and keep the array in memory)
-    const double f = t16::sel(q == 0, a[4 * j], t16::sel(q == 1, a[4 * j + 1], t16::sel(q == 2, a[4 * j + 2], a[4 * j + 3])));
-    v.put(g0 + r, g0 + q + 4 * j, f);
-  }
-#pragma unroll
-  for (int j = 0; j < 4; j++) Li[(q + 4 * j) * LL + r] = x[j];
+  for (int r = 0; r < 4; r++) v.put(g0 + li, g0 + lk + 4 * r, f.re[r]);
   return -1;
 }
 
@@ -110,7 +105,7 @@ potrf_batched_kernel(int count, const int *nvec, const long *offs, const int *or
     const int n = nvec[idx];
     const View<ST, LOWER> v{A + offs[idx], n};
     const int np = (n + LEAF - 1) / LEAF;
-    double logpart = 0.0;  // wave 0, lanes 0..15: sum of log(L_rr^2) of row r of every leaf
+    double logpart = 0.0;  // wave 0, diagonal lanes: sum of log(L_rr^2) of their row of every leaf
     int bad = -1;
     // Leaf p + 1 is factored by wave 0 during step p's trailing update
     // (look-ahead), from the tile (p + 1, p + 1) it updates itself; step
@@ -158,9 +153,9 @@ potrf_batched_kernel(int count, const int *nvec, const long *offs, const int *or
         }
         t16::acc_store(acc, Dg, LL);  // element (row, col) at col LL + row
         t16::wave_lds_fence();
-        double a[LEAF];
-        t16::static_for<0, LEAF>([&](auto C) { a[decltype(C)::value] = Dg[decltype(C)::value * LL + li]; });
-        const int b = leaf_step<ST, LOWER>(a, v, D * LEAF, Li, logpart);
+        TileAcc<double> f;
+        t16::frag_load(f, Dg, LL);
+        const int b = leaf_step<ST, LOWER>(f, v, D * LEAF, Li, logpart);
         if (lane == 0) flag = b;
       } else if (m > 0 && p >= 0) {
         // the other trailing tiles (I, J), p < J <= I, without (p+1, p+1),
@@ -278,7 +273,7 @@ potrf_batched_kernel(int count, const int *nvec, const long *offs, const int *or
       }
     }
     if (wave == 0) {
-      double logsum = logpart;  // lanes 16..63 hold 0
+      double logsum = logpart;  // the other lanes hold 0
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) logsum += __shfl_xor(logsum, off, 64);
       if (lane == 0) {
@@ -351,25 +346,20 @@ __device__ __forceinline__ void tile_update(v4d &T, const double *PI, const doub
     T = __builtin_amdgcn_mfma_f64_16x16x4f64(PJ[r * 4 * LL + lo], PI[r * 4 * LL + lo], T, 0, 0, kNegA);
 }
 
-// The leaf wave's step: factor the leaf at g0 (rows in a[], lane r + 16 q
-// holds row r), write L_pp to the matrix, 1 / L_rr (rows below n) to
-// rpiv[g0 + r] and inv(L_pp) to Li; returns the failing pivot's column
-// (g0 + k) or -1.
+// The leaf wave's step: factor the leaf at g0 held in f (row fragments), write
+// L_pp to the matrix, 1 / L_rr to rpiv[g0 + r] and inv(L_pp)
+// to Li; returns the failing pivot's column (g0 + k) or -1.
 template <typename ST, bool LOWER>
-__device__ __forceinline__ int leaf_step_piv(double (&a)[LEAF], const View<ST, LOWER> &v, int g0, double *Li,
+__device__ __forceinline__ int leaf_step_piv(TileAcc<double> &f, const View<ST, LOWER> &v, int g0, double *Li,
                                              double *rpiv) {
-  const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-  double x[4], rp;
-  const int b = t16::leaf_factor_invert<double>(a, x, rp);
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int b = t16::leaf_factor_invert<double>(f, [&](int r, double, double x) {
+    Li[li * LL + lk + 4 * r] = x;
+    if (lk + 4 * r == li) rpiv[g0 + li] = x;  // X(r, r) = 1 / L_rr (rpiv has whole leaves)
+  });
   if (b >= 0) return g0 + b;
-  if (q == 0 && g0 + r < v.n) rpiv[g0 + r] = rp;
 #pragma unroll
-  for (int j = 0; j < 4; j++) {  // lane group q writes columns q + 4 j of its row
-    const double f = t16::sel(q == 0, a[4 * j], t16::sel(q == 1, a[4 * j + 1], t16::sel(q == 2, a[4 * j + 2], a[4 * j + 3])));
-    v.put(g0 + r, g0 + q + 4 * j, f);
-  }
-#pragma unroll
-  for (int j = 0; j < 4; j++) Li[(q + 4 * j) * LL + r] = x[j];
+  for (int r = 0; r < 4; r++) v.put(g0 + li, g0 + lk + 4 * r, f.re[r]);
   return -1;
 }
 
@@ -464,9 +454,9 @@ potrf_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
       for (int D = 0; D < np; D++) {
         int b = -2;
         if (wave_wait([&] { return lds_acquire(&dready) == D; })) {
-          double a[LEAF];
-          t16::static_for<0, LEAF>([&](auto C) { a[decltype(C)::value] = Dg[decltype(C)::value * LL + li]; });
-          b = leaf_step_piv<ST, LOWER>(a, v, D * LEAF, Li + (D & 1) * LEAF * LL, rpiv);
+          TileAcc<double> f;
+          t16::frag_load(f, Dg, LL);
+          b = leaf_step_piv<ST, LOWER>(f, v, D * LEAF, Li + (D & 1) * LEAF * LL, rpiv);
         }
         if (lane == 0) {
           if (b != -1) {

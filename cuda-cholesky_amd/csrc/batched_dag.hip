@@ -287,31 +287,30 @@ __device__ void store_ainv_tile(double *D, int n, int i, int j, const double *P)
 // ---------------------------------------------------------------------------
 
 // P: lower 64 x 64 block (column-major, ld LD), factored in place.  Returns
-// the first failing column (0-based, every thread) or -1; in wave 0, lane r
-// (r < 16) accumulates log L_kk^2 of the rows k = r mod 16 below kvalid into
-// logsum (sum the wave's lanes for the block's total).
+// the first failing column (0-based, every thread) or -1; in wave 0 the lanes
+// on a leaf's diagonal accumulate log L_kk^2 of their rows k below kvalid
+// into logsum (sum the wave's lanes for the block's total).
 __device__ int lds_potrf64(double *P, double *Li, int *flag, int kvalid, double &logsum) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
 #pragma unroll 1
   for (int p = 0; p < TB / LEAF; p++) {
     const int g0 = p * LEAF;
     if (wave == 0) {
-      double a[LEAF];  // row li of the leaf
-      t16::static_for<0, LEAF>([&](auto C) { a[decltype(C)::value] = P[(g0 + decltype(C)::value) * LD + g0 + li]; });
-      double x[4], rpiv;
-      const int b = t16::leaf_factor_invert<double>(a, x, rpiv);
+      TileAcc<double> f;
+      t16::frag_load(f, P + g0 * LD + g0, LD);
+      double rp = 1.0;  // X(k, k) = 1 / L_kk in the lane on the diagonal
+      const int b = t16::leaf_factor_invert<double, true>(f, [&](int r, double, double x) {
+        Li[li * LL + lk + 4 * r] = x;
+        if (lk + 4 * r == li) rp = x;
+      });
       if (b < 0) {
-        // log of this lane's own pivot L_rr^2 = -2 log(1 / L_rr), off the pivot chain
-        if (lk == 0 && g0 + li < kvalid) logsum -= 2.0 * log(rpiv);
+        // log L_kk^2 = -2 log(1 / L_kk), off the pivot chain
+        if (lk == (li & 3) && g0 + li < kvalid) logsum -= 2.0 * log(rp);
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++) {  // lane group lk writes columns lk + 4 jj of row li
-          const double f = t16::sel(lk == 0, a[4 * jj], t16::sel(lk == 1, a[4 * jj + 1],
-                                    t16::sel(lk == 2, a[4 * jj + 2], a[4 * jj + 3])));
-          const int c = lk + 4 * jj;
-          P[(g0 + c) * LD + g0 + li] = c <= li ? f : 0.0;
+        for (int r = 0; r < 4; r++) {
+          const int c = lk + 4 * r;
+          P[(g0 + c) * LD + g0 + li] = c <= li ? f.re[r] : 0.0;
         }
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) Li[(lk + 4 * jj) * LL + li] = x[jj];
       }
       if (lane == 0) *flag = b < 0 ? -1 : g0 + b;
     }

@@ -281,9 +281,8 @@ __device__ __forceinline__ void diag_reciprocals(const T *S, T *dinv, int n) {
 // Blocked factor + inverse of one diagonal block (diag_potrf).
 //
 // The block is split into 16-column leaves.  Leaf p is factored and inverted
-// by one wave entirely in registers (lane r + 16 q holds row r, columns
-// q + 4 j) with cross-lane shuffles, so its 16 sequential pivots need no
-// workgroup barrier.  Everything else is 16 x 16 x 16 tile products on the
+// by one wave entirely in registers (leaf_factor_invert), so its 16
+// sequential pivots need no workgroup barrier.  Everything else is 16 x 16 x 16 tile products on the
 // matrix cores spread over the eight waves: the panel below the leaf
 // (L_Ip = A_Ip inv(L_pp)^H), the trailing update (A_IJ -= L_Ip L_Jp^H), and
 // the inverse X = inv(L) row block by row block as the factor's rows
@@ -295,57 +294,16 @@ using t16::TileAcc;
 using t16::acc_zero;
 using t16::acc_load;
 using t16::acc_store;
+using t16::acc_get;
+using t16::acc_rank4_sub;
+using t16::frag_load;
+using t16::frag_rank4;
+using t16::frag_store;
+using t16::leaf_factor_invert;
 using t16::tile_mma;
 using t16::wave_lds_fence;
 
 constexpr int BLK_THREADS = 512;
-
-// One wave factors the 16 x 16 leaf at S (leading dimension ls), writes the
-// factor straight to its place in the global matrix (rows and columns
-// g0 .. g0 + 15 of the n x n block at A, lower form: A(r, c) when lower,
-// conj into A(c, r) when upper; padding beyond n is not written) and
-// overwrites the leaf with its inverse (lower, zeros above).  Returns the
-// first non-positive / NaN pivot (0-based) or -1; on failure nothing is
-// written.
-template <typename T, typename ST>
-__device__ __forceinline__ int leaf_factor_inverse(T *S, int ls, bool lower, int n, int g0, ST *A,
-                                                long lda) {
-  int l = threadIdx.x & 63;
-  asm volatile("" : "+v"(l));  // lane-derived values computed here, not kept live across the kernel's loop
-  const int r = l & 15, q = l >> 4;
-  T a[LEAF];  // row r (row layout: the four lane groups hold the same row)
-#pragma unroll
-  for (int c = 0; c < LEAF; c++) a[c] = S[c * ls + r];
-  T x[4];
-  int bad;
-  if constexpr (is_complex<T>::value) {
-    // complex: factor and invert one after the other (the fused pass and the
-    // inverse-row accumulator of the caller do not fit the registers together)
-    double unused = 0.0;
-    bad = t16::leaf_factor_rows<T>(a, 0, &unused);
-    if (bad < 0) t16::leaf_inverse_cols<T>(a, x);
-  } else {
-    double rpiv;
-    bad = t16::leaf_factor_invert<T>(a, x, rpiv);
-  }
-  if (bad >= 0) return bad;
-  // lane group q writes columns q + 4 j of its row
-  auto pick = [&](const T *v, int j) {
-    return sel(q == 0, v[4 * j], sel(q == 1, v[4 * j + 1], sel(q == 2, v[4 * j + 2], v[4 * j + 3])));
-  };
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int c = q + 4 * j, gr = g0 + r, gc = g0 + c;
-    const T v = pick(a, j);
-    if (r >= c && gr < n) {
-      if (lower) A[(long)gc * lda + gr] = convert<ST>(v);
-      else A[(long)gr * lda + gc] = convert<ST>(conjx(v));
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; j++) S[(q + 4 * j) * ls + r] = x[j];
-  return -1;
-}
 
 // LDS holds only the lower-triangle tiles, packed: tile (I, J), I >= J, at
 // index I (I + 1) / 2 + J, each 16 x 16 column-major with leading dimension
@@ -362,184 +320,299 @@ __device__ __forceinline__ int leaf_factor_inverse(T *S, int ls, bool lower, int
 template <typename T>
 constexpr int diag_waves_per_eu() { return is_complex<T>::value ? 2 : 4; }
 
-// Factor and invert the lower-form block held in S (the packed tiles above,
-// already loaded, identity padding beyond n; `flag` an LDS word).  The factor
-// goes to A (lower form: A(r, c), or conj into A(c, r) when !lower) and
-// inv(L) densely to W (ld ldw, zeros above the diagonal, n x n only).
-// Returns -1, or the first non-positive / NaN pivot (0-based, the same value
-// in every thread; the factor is then only partly written).
-// EARLY: wave 0 has written tile (0, 0) itself and set flag = -1, and the
-// other waves may still be filling the rest of S (leaf 0 overlaps their loads;
-// the barrier after it completes S).
-template <typename T, typename ST, int NMAX, bool EARLY = false>
-__device__ __forceinline__ int diag_block_factor(T *S, int &flag, int lower, int n, ST *A, long lda, ST *W,
-                                                 long ldw) {
-  constexpr int NPMAX = NMAX / LEAF, LL = LEAF + 1, TS = LEAF * LL, NW = BLK_THREADS / 64;
-  static_assert(NPMAX <= NW, "each wave finishes at most one tile of a row of the inverse");
-  const int tid = threadIdx.x, wave = tid >> 6;
-  const int np = (n + LEAF - 1) / LEAF;
-  auto tile = [&](int I, int J) { return S + (I * (I + 1) / 2 + J) * TS; };
-  auto elem = [&](int r, int c) -> T & { return tile(r / LEAF, c / LEAF)[(c % LEAF) * LL + r % LEAF]; };
-  if constexpr (!EARLY) {
-    if (tid == 0) flag = -1;
-    __syncthreads();
-  }
-  // One leaf of look-ahead: while wave 0 updates tile (p+1, p+1) and factors
-  // leaf p + 1, waves 1 .. NW-1 apply the rest of step p's trailing update
-  // and form S_{p+1,J} = sum_{K=J..p} L_{p+1,K} X_KJ (wave 1 + J) for row
-  // p + 1 of X = inv(L).  At the start of step p + 1 (phase A) the same wave
-  // writes L_{p+1,J} to A and finishes X_{p+1,J} = -X_{p+1,p+1} S_{p+1,J} in
-  // its tile (L X = I row by row), beside the panel solves below leaf p + 1:
-  // the inverse is complete when the last leaf is, with no pass of its own.
-  // Step p = -1 only factors leaf 0 (one call site keeps the leaf inlined once).
-  TileAcc<T> sacc;  // S_{p+1, wave-1}, carried from phase B to the next phase A
-  acc_zero(sacc);
-  for (int p = -1; p < np; p++) {
-    if (p >= 0) {
-      // phase A: panel item k (L_Ip = A_Ip X_pp^H, I = p + 1 + k) on wave 0
-      // (k = 0) or wave p + k; row p of the inverse on waves 1 .. p
-      const int k = wave == 0 ? 0 : (wave > p ? wave - p : -1);
-      if (k >= 0 && p + 1 + k < np) {
-        const int I = p + 1 + k;
-        TileAcc<T> acc;
-        acc_zero(acc);
-        tile_mma<true>(acc, tile(I, p), LL, tile(p, p), LL, 1.0);
-        acc_store(acc, tile(I, p), LL);
-      }
-      if (wave >= 1 && wave <= p) {
-        const int J = wave - 1;
-        T *tpj = tile(p, J);
-        {  // L_pJ to its place in A (lower form; padding rows are not written)
-          const int l = tid & 63, rr = l & 15, cq = l >> 4, r = p * LEAF + rr;
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const int c = J * LEAF + cq + 4 * j;
-            const T v = tpj[(cq + 4 * j) * LL + rr];
-            if (r < n) {
-              if (lower) A[(long)c * lda + r] = convert<ST>(v);
-              else A[(long)r * lda + c] = convert<ST>(conjx(v));
-            }
-          }
-        }
-        wave_lds_fence();
-        acc_store(sacc, tpj, LL);
-        wave_lds_fence();
-        TileAcc<T> acc;
-        acc_zero(acc);
-        tile_mma<false>(acc, tile(p, p), LL, tpj, LL, -1.0);
-        wave_lds_fence();
-        acc_store(acc, tpj, LL);
-      }
-      __syncthreads();
-    }
-    if (p + 1 < np) {
-      if (wave == 0) {  // A_{p+1,p+1} -= L_{p+1,p} L_{p+1,p}^H, then leaf p + 1
-        if (p >= 0) {
-          TileAcc<T> acc;
-          acc_load(acc, tile(p + 1, p + 1), LL);
-          tile_mma<true>(acc, tile(p + 1, p), LL, tile(p + 1, p), LL, -1.0);
-          acc_store(acc, tile(p + 1, p + 1), LL);
-          wave_lds_fence();
-        }
-        const int bad = leaf_factor_inverse<T, ST>(tile(p + 1, p + 1), LL, lower, n, (p + 1) * LEAF, A, lda);
-        if (bad >= 0 && (tid & 63) == 0) flag = (p + 1) * LEAF + bad;
-      } else if (p >= 0) {
-        int t = 0;
-        for (int J = p + 1; J < np; J++)
-          for (int I = (J == p + 1) ? J + 1 : J; I < np; I++, t++)
-            if (t % (NW - 1) == wave - 1) {  // A_IJ -= L_Ip L_Jp^H
-              TileAcc<T> acc;
-              acc_load(acc, tile(I, J), LL);
-              tile_mma<true>(acc, tile(I, p), LL, tile(J, p), LL, -1.0);
-              acc_store(acc, tile(I, J), LL);
-            }
-        if (wave - 1 <= p) {  // S_{p+1,J}, J = wave - 1: row p + 1 of L is complete
-          const int J = wave - 1;
-          acc_zero(sacc);
-          for (int K = J; K <= p; K++) tile_mma<false>(sacc, tile(p + 1, K), LL, tile(K, J), LL, 1.0);
-        }
-      }
-    }
-    __syncthreads();
-    const int f = flag;
-    if (f >= 0) return f;  // leaf p + 1 failed (padding never fails, so f < n)
-  }
-  // W = inv(L) dense, zeros above the diagonal
-  for_block<NMAX, BLK_THREADS>(n, [&](int r, int c) {
-    W[(long)c * ldw + r] = convert<ST>(r >= c ? elem(r, c) : from_real<T>(0.0));
-  });
-  return -1;
+// Elements of LDS that the factorisation of a diagonal block of order NMAX
+// uses: the packed tiles and a buffer for the leaf's factor.
+template <int NMAX>
+constexpr int diag_lds_elems() {
+  constexpr int NP = NMAX / LEAF;
+  return (NP * (NP + 1) / 2 + 1) * LEAF * (LEAF + 1);
 }
 
-// Bytes of the packed lower-triangle tiles of a diagonal block of order NMAX.
-template <typename T, int NMAX>
-constexpr int diag_tiles_bytes() {
-  return (NMAX / LEAF) * (NMAX / LEAF + 1) / 2 * LEAF * (LEAF + 1) * (int)sizeof(T);
+// Factor and invert the lower-form block of order n whose tiles src delivers
+// (src.load<LO, HI>(I, x): the stored values of tiles (I, LO .. HI-1);
+// src.fix(x, r, c): the value of an element, identity beyond n) with S as
+// workspace (`flag` an LDS word).  The factor goes to A (lower form: A(r, c),
+// or conj into A(c, r) when !lower) and inv(L) to the lower tiles of W (ld ldw,
+// n x n only, zeros above the diagonal of the diagonal tiles; with ZEROS also
+// in the tiles above them).  Nothing is done when `failed`.  Returns -1,
+// or the first non-positive / NaN pivot (0-based, the same value in every
+// thread; the factor is then only partly written).
+//
+// Wave 0 factors the leaves; workers 0 .. NW-2 are the other waves.  Worker w
+// holds tile row w + 2 of the trailing matrix in registers, as row fragments
+// (at once matrix-core operands and results).  Step p, after leaf p:
+//   phase A: wave 0 forms the panel tile (p+1, p), worker w >= p the panel tile
+//     (w+2, p), L_Ip = A_Ip X_pp^H; worker J < p finishes tile J of row p of
+//     X = inv(L), X_pJ = -X_pp S_pJ (L X = I row by row);
+//   phase B: wave 0 updates tile (p+1, p+1) and factors leaf p + 1; worker
+//     w >= p applies step p to its row, and the owner of row p + 2 hands tiles
+//     (p+2, p+1) and (p+2, p+2) to wave 0 through LDS; worker J <= p forms
+//     S_{p+1,J} = sum_{K=J..p} L_{p+1,K} X_KJ.  Tiles of L and X finished in
+//     phase A are written to A and W here.
+// The inverse is complete with the last leaf, with no pass of its own.  Step
+// p = -1 only factors leaf 0 (one call site keeps the leaf inlined once).
+//
+// The time is the chain leaf -> panel tile (p+1, p) -> update of tile
+// (p+1, p+1) -> leaf in wave 0, so that wave does nothing else, and wave 4, on
+// the same SIMD, is worker 6, which has no row; the workers, at a lower issue
+// priority, keep up with it because a row in registers leaves one LDS operand
+// per product.  One CU takes about 10000 cycles to read the block from HBM
+// (longer than two leaves): leaf 0 overlaps the left half of every row, leaf 1
+// the right half.  One 128 x 128 double
+// block alone: 24.5 us between events (36 us with a column-by-column leaf in a
+// layout of its own, the tiles in LDS, the write-out in wave 0 and the block
+// loaded element by element).
+template <typename T, typename ST, int NMAX, bool ZEROS, typename Src>
+__device__ __forceinline__ int diag_block_factor(const Src &src, bool failed, T *S, int &flag, int lower, int n,
+                                                 ST *A, long lda, ST *W, long ldw) {
+  constexpr int NPMAX = NMAX / LEAF, LL = LEAF + 1, TS = LEAF * LL, NW = BLK_THREADS / 64;
+  static_assert(NPMAX <= NW && NW == 8, "a worker per tile of a row of the inverse; wave 4 shares wave 0's SIMD");
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int np = (n + LEAF - 1) / LEAF;
+  int lane = tid & 63;
+  asm volatile("" : "+v"(lane));
+  const int lc = lane & 15, lg = lane >> 4;
+  auto tile = [&](int I, int J) { return S + (I * (I + 1) / 2 + J) * TS; };
+  T *const Lbuf = S + NPMAX * (NPMAX + 1) / 2 * TS;  // L_pp
+  // row fragments f of L_IJ to A, of X_IJ to W (entries above the diagonal of
+  // a diagonal tile: not written, zero)
+  auto put_a = [&](const TileAcc<T> &f, int I, int J) {
+    const int r = I * LEAF + lc, c0 = J * LEAF + lg;
+    if (r < n) {
+      ST *a = lower ? A + (long)c0 * lda + r : A + (long)r * lda + c0;
+      const long step = lower ? 4 * lda : 4;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        if (r >= c0 + 4 * j) *a = lower ? convert<ST>(acc_get(f, j)) : convert<ST>(conjx(acc_get(f, j)));
+        a += step;
+      }
+    }
+  };
+  auto put_w = [&](const TileAcc<T> &f, int I, int J) {
+    const int r = I * LEAF + lc, c0 = J * LEAF + lg;
+    if (r < n) {
+      ST *w = W + (long)c0 * ldw + r;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        if (c0 + 4 * j < n) *w = convert<ST>(acc_get(f, j));
+        w += 4 * ldw;
+      }
+    }
+  };
+  // The two roles are disjoint code (the register budget is the larger of
+  // them) with the same barriers: one after phase A, one after phase B.
+  if (wave == 0) {
+    __builtin_amdgcn_s_setprio(3);  // issue ahead of the workers and of any other kernel's waves
+    typename Src::V x0[NPMAX][4], x1[NPMAX][4];
+    const bool row1 = np > 1;
+    src.template load<0, 1>(0, x0);
+    if (row1) src.template load<0, 2>(1, x1);
+    if (failed) return -1;
+    if (tid == 0) flag = -1;
+    TileAcc<T> fd, fl;  // the diagonal tile to factor, panel tile (p+1, p)
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc_set(fd, j, src.fix(x0[0][j], lc, lg + 4 * j));
+    if (row1) {
+#pragma unroll
+      for (int J = 0; J < 2; J++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc_set(fl, j, src.fix(x1[J][j], LEAF + lc, J * LEAF + lg + 4 * j));
+        frag_store(fl, tile(1, J), LL);
+      }
+    }
+    for (int p = -1; p < np - 1; p++) {
+      if (p >= 0) {
+        TileAcc<T> xf, af;
+        frag_load(xf, tile(p, p), LL);
+        frag_load(af, tile(p + 1, p), LL);
+        frag_load(fd, tile(p + 1, p + 1), LL);
+        acc_zero(fl);
+#pragma unroll
+        for (int s = 0; s < 4; s++) frag_rank4<false>(fl, acc_get(af, s), acc_get(xf, s));
+        frag_store(fl, tile(p + 1, p), LL);
+#pragma unroll
+        for (int s = 0; s < 4; s++) frag_rank4<true>(fd, acc_get(fl, s), acc_get(fl, s));
+        __syncthreads();
+      }
+      T *const xt = tile(p + 1, p + 1) + lc * LL + lg, *const lt = Lbuf + lg * LL + lc;
+      const int bad = leaf_factor_invert<T>(fd, [&](int r, T l, T x) {
+        lt[4 * r * LL] = l;
+        xt[4 * r] = x;
+      });
+      if (bad >= 0 && lane == 0) flag = (p + 1) * LEAF + bad;
+      __syncthreads();
+      if (bad >= 0) return (p + 1) * LEAF + bad;  // padding never fails, so this is below n
+    }
+    put_a(fd, np - 1, np - 1);
+    frag_load(fl, tile(np - 1, np - 1), LL);
+    put_w(fl, np - 1, np - 1);
+    return -1;
+  }
+
+  __builtin_amdgcn_s_setprio(2);
+  const int wk = wave == 4 ? NW - 2 : (wave < 4 ? wave - 1 : wave - 2);  // worker
+  const int row = wk + 2 < np ? wk + 2 : -1;
+  TileAcc<T> R[NPMAX];  // the worker's tile row
+  constexpr int HALF = NPMAX * 6 / 8;
+  // its tiles LO .. HI - 1
+  auto take = [&](auto lo, auto hi) __attribute__((always_inline)) {
+    constexpr int LO = decltype(lo)::value, HI = decltype(hi)::value;
+    typename Src::V x[NPMAX][4];
+    src.template load<LO, HI>(row, x);
+    if (failed) return;
+    t16::static_for<LO, HI>([&](auto Jc) {
+      constexpr int J = decltype(Jc)::value;
+      if (J <= row) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc_set(R[J], j, src.fix(x[J][j], row * LEAF + lc, J * LEAF + lg + 4 * j));
+      }
+    });
+  };
+  take(std::integral_constant<int, 0>{}, std::integral_constant<int, HALF>{});
+  if (failed) return -1;
+  __syncthreads();
+  TileAcc<T> sacc;  // S_{p+1,wk}, carried from phase B to the next phase A
+  TileAcc<T> lp;    // the panel tile, or tile wk of row p of L
+  acc_zero(sacc);
+  int zi = -1, zj = 1;  // worker NW - 2: tile above the diagonal last zeroed in W
+  // panel tile (row, J), J = p; worker NW - 2, which has no tile before the
+  // last row, takes L_pp instead
+  auto panel = [&](auto Jc) __attribute__((always_inline)) {
+    constexpr int J = decltype(Jc)::value;
+    TileAcc<T> xf, acc;
+    frag_load(xf, tile(J, J), LL);
+    acc_zero(acc);
+#pragma unroll
+    for (int s = 0; s < 4; s++) frag_rank4<false>(acc, acc_get(R[J], s), acc_get(xf, s));
+    frag_store(acc, tile(row, J), LL);
+    lp = acc;
+  };
+  if (row > 0) panel(std::integral_constant<int, 0>{});
+  if (wk == NW - 2 && np > 1) frag_load(lp, Lbuf, LL);
+  int bad = flag;  // of leaf p (padding never fails, so it is below n)
+  if (bad >= 0) return bad;
+  if (np > 1) __syncthreads();
+  take(std::integral_constant<int, HALF>{}, std::integral_constant<int, NPMAX>{});
+  for (int p = 0;; p++) {
+    // phase B of step p
+    if (wk >= p && row > 0) {  // A_IJ -= L_Ip L_Jp^H, I = row
+      t16::static_for<1, NPMAX>([&](auto Jc) {
+        constexpr int J = decltype(Jc)::value;
+        if (J > p && J <= row) {
+          TileAcc<T> b = lp;
+          if (J < row) frag_load(b, tile(J, p), LL);
+#pragma unroll
+          for (int s = 0; s < 4; s++) frag_rank4<true>(R[J], acc_get(lp, s), acc_get(b, s));
+          if (row == p + 2) frag_store(R[J], tile(row, J), LL);
+        }
+      });
+    } else if (wk < p || (wk == NW - 2 && p < np - 1)) {
+      const int J = wk < p ? wk : p;
+      put_a(lp, p, J);
+      TileAcc<T> x;
+      frag_load(x, tile(p, J), LL);
+      put_w(x, p, J);
+    }
+    if (p == np - 1) return -1;
+    if (ZEROS && wk == NW - 2) {  // zeros of W above the diagonal tiles: its NPMAX / 2 next ones
+      for (int u = 0; u < NPMAX / 2; u++) {
+        if (++zi >= zj) {
+          zi = 0;
+          zj++;
+        }
+        if (zj >= np) break;
+        ST *w = W + (long)(zj * LEAF + lg) * ldw + zi * LEAF + lc;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (zj * LEAF + lg + 4 * j < n) w[j * 4 * ldw] = convert<ST>(from_real<T>(0.0));
+      }
+    }
+    if (wk <= p) {  // S_{p+1,wk}: row p + 1 of L is complete
+      acc_zero(sacc);
+      for (int K = wk; K <= p; K++) tile_mma<false>(sacc, tile(p + 1, K), LL, tile(K, wk), LL, 1.0);
+    }
+    __syncthreads();
+    // phase A of step q
+    const int q = p + 1;
+    if (wk >= q && row > 0) {
+      t16::static_for<1, NPMAX>([&](auto Jc) {
+        if (decltype(Jc)::value == q) panel(Jc);
+      });
+    } else if (wk < q) {
+      T *tqj = tile(q, wk);
+      TileAcc<T> xf, acc;
+      frag_load(xf, tile(q, q), LL);
+      frag_load(lp, tqj, LL);
+      acc_zero(acc);
+#pragma unroll
+      for (int s = 0; s < 4; s++) acc_rank4_sub(acc, acc_get(xf, s), acc_get(sacc, s));
+      acc_store(acc, tqj, LL);
+      wave_lds_fence();
+    }
+    if (wk == NW - 2 && q < np - 1) frag_load(lp, Lbuf, LL);
+    bad = flag;
+    if (bad >= 0) return bad;
+    if (q < np - 1) __syncthreads();
+  }
 }
+
+// Tiles of the n x n block at A in global memory, lower form.
+template <typename T, typename ST>
+struct GlobalTiles {
+  using V = ST;
+  const ST *A;
+  long lda;
+  int lower, n;
+  // x[J][j] <- this lane's elements of tile (I, J), LO <= J < HI and J <= I
+  // (row fragments), all loads in flight together; beyond n from a clamped
+  // (always valid) address, selected away by fix.  A block of whole tiles
+  // walks one pointer, without the clamps and 64-bit index products.
+  template <int LO, int HI, int NP>
+  __device__ __forceinline__ void load(int I, V (&x)[NP][4]) const {
+    const int lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4, r = I * LEAF + lc;
+    if (LO > I) return;
+    if (n % LEAF == 0) {
+      const ST *a = lower ? A + (long)(LO * LEAF + lg) * lda + r : A + (long)r * lda + LO * LEAF + lg;
+      const long step = lower ? 4 * lda : 4;
+      t16::static_for<LO, HI>([&](auto Jc) {
+        constexpr int J = decltype(Jc)::value;
+        if (J <= I) {
+#pragma unroll
+          for (int j = 0; j < 4; j++, a += step) x[J][j] = *a;
+        }
+      });
+    } else {
+      const int rc = min(r, n - 1);
+      t16::static_for<LO, HI>([&](auto Jc) {
+        constexpr int J = decltype(Jc)::value;
+        if (J <= I) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const int c = min(J * LEAF + lg + 4 * j, n - 1);
+            x[J][j] = lower ? A[(long)c * lda + rc] : A[(long)rc * lda + c];
+          }
+        }
+      });
+    }
+  }
+  // the value of element (r, c) loaded as x, identity beyond n
+  __device__ __forceinline__ T fix(ST x, int r, int c) const {
+    const T v = lower ? convert<T>(x) : conjx(convert<T>(x));
+    if (n % LEAF == 0) return v;
+    return t16::sel(r < n && c < n, v, from_real<T>(r == c ? 1.0 : 0.0));
+  }
+};
 
 template <typename T, typename ST, int NMAX>
 __global__ void __launch_bounds__(BLK_THREADS)
 __attribute__((amdgpu_waves_per_eu(diag_waves_per_eu<T>(), diag_waves_per_eu<T>())))
 diag_potrf_kernel(int lower, int n, ST *A, long lda, ST *W, long ldw, int *info, long info_off) {
-  if (*info != 0) return;
-  // This block is on the critical path of the factorisation while trailing-
-  // update waves share its SIMDs: take instruction issue ahead of them.
-  __builtin_amdgcn_s_setprio(3);
-  constexpr int NPMAX = NMAX / LEAF, LL = LEAF + 1, TS = LEAF * LL;
-  __shared__ T S[NPMAX * (NPMAX + 1) / 2 * TS];
+  __shared__ T S[diag_lds_elems<NMAX>()];
   __shared__ int flag;
-  const int tid = threadIdx.x;
-  const int np = (n + LEAF - 1) / LEAF, npad = np * LEAF;
-  auto tile = [&](int I, int J) { return S + (I * (I + 1) / 2 + J) * TS; };
-  auto elem = [&](int r, int c) -> T & { return tile(r / LEAF, c / LEAF)[(c % LEAF) * LL + r % LEAF]; };
-  if (tid < 64) {
-    // wave 0: tile (0, 0) only (lower form, identity padding), then leaf 0
-    // at once while the other waves load the rest of the block
-    const int rr = tid & 15, cq = tid >> 4, rc = min(rr, n - 1);
-    T v[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int cc = min(cq + 4 * j, n - 1);
-      const ST x = lower ? A[(long)cc * lda + rc] : A[(long)rc * lda + cc];
-      v[j] = lower ? convert<T>(x) : conjx(convert<T>(x));
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int c = cq + 4 * j;
-      if (rr >= c) tile(0, 0)[c * LL + rr] = (rr < n && c < n) ? v[j] : from_real<T>(rr == c ? 1.0 : 0.0);
-    }
-    if (tid == 0) flag = -1;
-    wave_lds_fence();
-  } else {
-    // waves 1 .. 7: identity padding and the lower form of every other tile,
-    // read along memory's contiguous index (i), every load of a thread in
-    // flight at once (clamped, always valid addresses)
-    constexpr int T2 = BLK_THREADS - 64, U = (NMAX * NMAX + T2 - 1) / T2;
-    const int t2 = tid - 64;
-    for (int c = t2; c < npad; c += T2)
-      for (int r = max(n, c); r < npad; r++)
-        if (r >= LEAF || c >= LEAF) elem(r, c) = from_real<T>(r == c ? 1.0 : 0.0);
-    // in batches that fit the registers (one for 4-byte data, two for 8-byte)
-    constexpr int NB = sizeof(ST) > 4 ? 2 : 1, UB = (U + NB - 1) / NB;
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-      ST x[UB];
-#pragma unroll
-      for (int u = 0; u < UB; u++) {
-        const int e = min(t2 + T2 * (b * UB + u), NMAX * NMAX - 1), i = e % NMAX, k = e / NMAX;
-        x[u] = A[(long)min(k, n - 1) * lda + min(i, n - 1)];
-      }
-#pragma unroll
-      for (int u = 0; u < UB; u++) {
-        const int e = t2 + T2 * (b * UB + u), i = e % NMAX, k = e / NMAX;
-        const int r = lower ? i : k, c = lower ? k : i;  // lower form, r >= c wanted
-        if (b * UB + u < U && e < NMAX * NMAX && i < n && k < n && r >= c && (r >= LEAF || c >= LEAF))
-          elem(r, c) = lower ? convert<T>(x[u]) : conjx(convert<T>(x[u]));
-      }
-    }
-  }
-  const int bad = diag_block_factor<T, ST, NMAX, true>(S, flag, lower, n, A, lda, W, ldw);
-  if (bad >= 0 && tid == 0) *info = (int)(info_off + bad + 1);
+  const int failed = *info;  // tested once the block's loads are issued
+  const GlobalTiles<T, ST> src{A, lda, lower, n};
+  const int bad = diag_block_factor<T, ST, NMAX, false>(src, failed != 0, S, flag, lower, n, A, lda, W, ldw);
+  if (bad >= 0 && threadIdx.x == 0) *info = (int)(info_off + bad + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -770,9 +843,29 @@ __device__ __forceinline__ void panel_publish(int *f, int epoch) {
 template <typename ST>
 constexpr int panel_lds_bytes() {
   constexpr int g = 4 * PK_B * PanelMma<ST>::LK * (int)sizeof(ST);
-  constexpr int d = diag_tiles_bytes<double, PK_B>();
+  constexpr int d = diag_lds_elems<PK_B>() * (int)sizeof(double);
   return g > d ? g : d;
 }
+
+// The packed lower tiles in LDS as the source of diag_block_factor, which
+// reads a tile before it overwrites it (each wave only the tiles it owns).
+struct LdsTiles {
+  using V = double;
+  const double *S;
+  template <int LO, int HI, int NP>
+  __device__ __forceinline__ void load(int I, double (&x)[NP][4]) const {
+    const int lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
+    t16::static_for<LO, HI>([&](auto Jc) {
+      constexpr int J = decltype(Jc)::value;
+      if (J <= I) {
+        const double *t = S + (I * (I + 1) / 2 + J) * LEAF * (LEAF + 1);
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[J][j] = t[(lg + 4 * j) * (LEAF + 1) + lc];
+      }
+    });
+  }
+  __device__ double fix(double x, int, int) const { return x; }
+};
 
 // ws: C inverses inv(L_JJ) (128 x 128, ld 128), then C partial sums (128 x 128).
 template <typename ST>
@@ -851,8 +944,10 @@ panel_potrf_kernel(int m, int jb, ST *A, long lda, ST *ws, int *flags, int epoch
       }
     });
   }
-  const int bad = diag_block_factor<T, ST, PK_B>(reinterpret_cast<T *>(lds_raw), sh_flag, 1, ra, Abb, lda,
-                                                 Winv + b * BB, PK_B);
+  __syncthreads();
+  T *const S = reinterpret_cast<T *>(lds_raw);
+  const int bad = diag_block_factor<T, ST, PK_B, true>(LdsTiles{S}, false, S, sh_flag, 1, ra, Abb, lda,
+                                                       Winv + b * BB, PK_B);
   if (bad >= 0) {
     if (threadIdx.x == 0) {
       int expected = 0;

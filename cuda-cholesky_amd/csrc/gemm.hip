@@ -583,6 +583,153 @@ hipError_t dispatch_ops(hipStream_t s, int ta, int tb, const KParams<T> &p, int 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Panel solve: A <- A W^H (lower, rows r0 .. r0 + R - 1 of a workgroup) or
+// A <- W A (upper, columns), W lower triangular of order ib <= IB, in place.
+// The launch is a link of the factorisation's chain (diagonal block, panel
+// solve, update, next diagonal block) with little work, so what bounds it is
+// latency: a whole strip of A and the workgroup's part of W are loaded at
+// once (A through LDS, W straight into operand fragments), one barrier, then
+// only products.  Strips of R = 16 rows (real) fill the chip up to 4096 rows;
+// beyond, and for complex, R = 32 halves the reads of W.  W's zero
+// triangle is skipped: 36 of 64 tile products (real).  Wave w takes the column
+// tiles w' and NT - 1 - w' (equal work), w' = w (real) or w / 2 with the row
+// tiles split between the two waves (complex: NT = 4).
+// 4000 x 128 doubles: 7.4 us per launch (median over a factorisation), 19 us as a 64 x 128 tile product with
+// W dense and K in steps of 16.
+// ---------------------------------------------------------------------------
+template <typename T, bool LOWER, int R>
+__global__ void __launch_bounds__(NTHREADS, 2) panel_solve_kernel(long m, int ib, T *A, long lda, const T *W, long ldw,
+                                                               const int *abort_flag) {
+  constexpr bool CPLX = is_complex<T>::value;
+  using RT = typename Prec<T>::R;
+  using V = typename Prec<T>::V;
+  constexpr int P = CPLX ? 2 : 1, IB = CPLX ? 64 : 128, NTL = IB / 16;
+  constexpr int WR = CPLX ? 2 : 1;                         // waves along the strip
+  static_assert(R >= 16 * WR, "a strip tile per wave");
+  constexpr int NR = R / 16 / WR;                          // strip tiles per wave
+  // strip in LDS: element (k, i), i along the strip; conflict-free fragment
+  // reads need the stride of lower strips (k-major) to be 16 mod 32 and that
+  // of upper ones (i-major) to be 2 mod 32
+  constexpr int LDK = LOWER ? 1 : IB + 2, LDI = LOWER ? (R == 16 ? 16 : R + 16) : 1;
+  constexpr int PLANE = LOWER ? IB * LDI : R * LDK;
+  __shared__ RT sA[P * PLANE];
+  auto at = [&](int k, int i) { return LOWER ? k * LDI + i : i * LDK + k; };
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lc = lane & 15, lg = lane >> 4, wr = wave % WR, wc = wave / WR;
+  const long i0 = (long)blockIdx.x * R;
+  const int failed = abort_flag != nullptr ? *abort_flag : 0;
+
+  // strip: clamped (always valid) addresses; what is beyond the edges is
+  // multiplied by zeros of W (k >= ib) or not stored (i >= m)
+  constexpr int E = R * IB / NTHREADS;
+  T ra[E];
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    const int k = LOWER ? tid / R + e * (NTHREADS / R) : tid % IB;
+    const int i = LOWER ? tid % R : tid / IB + e * (NTHREADS / IB);
+    const int kc = min(k, ib - 1);
+    const long ic = min(i0 + i, m - 1);
+    ra[e] = LOWER ? A[(long)kc * lda + ic] : A[ic * lda + kc];
+  }
+  // fragments of W's row tiles c = wc (k tiles 0 .. wc) and NTL - 1 - wc
+  T w[2][NTL][4];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int c = h == 0 ? wc : NTL - 1 - wc;
+#pragma unroll
+    for (int kt = 0; kt < NTL; kt++) {
+      if (h == 0 && kt >= NTL / 2) continue;  // c < NTL / 2
+      if (kt > c) continue;
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const int r = 16 * c + lc, k = 16 * kt + 4 * s + lg;
+        w[h][kt][s] = W[(long)min(k, ib - 1) * ldw + min(r, ib - 1)];
+      }
+    }
+  }
+  if (failed != 0) return;
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    const int k = LOWER ? tid / R + e * (NTHREADS / R) : tid % IB;
+    const int i = LOWER ? tid % R : tid / IB + e * (NTHREADS / IB);
+    lds_put(sA, PLANE, at(k, i), k < ib ? ra[e] : from_real<T>(0.0));
+  }
+  __syncthreads();
+
+  V acc[P][2][NR];
+#pragma unroll
+  for (int q = 0; q < P; q++)
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int i = 0; i < NR; i++) acc[q][h][i] = (V){0, 0, 0, 0};
+#pragma unroll
+  for (int kt = 0; kt < NTL; kt++) {
+    if (kt > NTL - 1 - wc) continue;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      RT ar[NR], ai[NR];
+#pragma unroll
+      for (int i = 0; i < NR; i++) {
+        const int idx = at(16 * kt + 4 * s + lg, 16 * (wr * NR + i) + lc);
+        ar[i] = sA[idx];
+        if constexpr (CPLX) ai[i] = sA[PLANE + idx];
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int c = h == 0 ? wc : NTL - 1 - wc;
+        if (h == 0 && kt >= NTL / 2) continue;
+        if (kt > c) continue;
+        // zero above the diagonal and beyond ib (selected, never multiplied)
+        const int r = 16 * c + lc, k = 16 * kt + 4 * s + lg;
+        const bool ok = k <= r && r < ib;
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+          // result: lane lc along memory's contiguous index (the strip for
+          // lower, W's rows for upper)
+          if constexpr (!CPLX) {
+            const RT b = ok ? w[h][kt][s] : RT(0);
+            acc[0][h][i] = LOWER ? mma(b, ar[i], acc[0][h][i]) : mma(ar[i], b, acc[0][h][i]);
+          } else {
+            const RT br = ok ? w[h][kt][s].x : RT(0), bi = ok ? w[h][kt][s].y : RT(0);
+            if constexpr (LOWER) {  // A conj(W)^T
+              acc[0][h][i] = mma(br, ar[i], acc[0][h][i]);
+              acc[0][h][i] = mma(bi, ai[i], acc[0][h][i]);
+              acc[1][h][i] = mma(br, ai[i], acc[1][h][i]);
+              acc[1][h][i] = mma(-bi, ar[i], acc[1][h][i]);
+            } else {  // W A
+              acc[0][h][i] = mma(ar[i], br, acc[0][h][i]);
+              acc[0][h][i] = mma(-ai[i], bi, acc[0][h][i]);
+              acc[1][h][i] = mma(ai[i], br, acc[1][h][i]);
+              acc[1][h][i] = mma(ar[i], bi, acc[1][h][i]);
+            }
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int c = h == 0 ? wc : NTL - 1 - wc;
+#pragma unroll
+    for (int i = 0; i < NR; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int it = 16 * (wr * NR + i), rr = res_row<T>(lg, r);
+        const long gi = i0 + it + (LOWER ? lc : rr);
+        const int gc = 16 * c + (LOWER ? rr : lc);
+        if (gi < m && gc < ib) {
+          T v;
+          if constexpr (CPLX) v = cmake<T>(acc[0][h][i][r], acc[1][h][i][r]);
+          else v = acc[0][h][i][r];
+          if (LOWER) A[(long)gc * lda + gi] = v;
+          else A[gi * lda + gc] = v;
+        }
+      }
+  }
+}
+
 template <typename T>
 __global__ void copy2d_kernel(int m, int n, const T *S, long lds, T *D, long ldd) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -655,6 +802,34 @@ hipError_t copy2d(hipStream_t s, long m, long n, const T *S, long lds, T *D, lon
   hipLaunchKernelGGL((copy2d_kernel<T>), grid, dim3(256), 0, s, (int)m, (int)n, S, lds, D, ldd);
   return hipGetLastError();
 }
+
+template <typename T>
+hipError_t panel_solve(hipStream_t s, bool lower, long m, int ib, T *A, long lda, const T *W, long ldw,
+                       const int *abort_flag) {
+  if (m <= 0 || ib <= 0) return hipSuccess;
+  if (ib > (is_complex<T>::value ? 64 : 128)) return hipErrorInvalidValue;
+  // one 16-row strip per CU while that fills at most the chip, else half as many
+  constexpr bool CPLX = is_complex<T>::value;
+  const int R = !CPLX && m <= 16 * 256 ? 16 : 32;
+  const dim3 grid((unsigned)((m + R - 1) / R));
+#define HC_PS(L, RR) \
+  hipLaunchKernelGGL((panel_solve_kernel<T, L, RR>), grid, dim3(NTHREADS), 0, s, m, ib, A, lda, W, ldw, abort_flag)
+  if constexpr (!CPLX) {
+    if (R == 16) {
+      if (lower) HC_PS(true, 16);
+      else HC_PS(false, 16);
+      return hipGetLastError();
+    }
+  }
+  if (lower) HC_PS(true, 32);
+  else HC_PS(false, 32);
+#undef HC_PS
+  return hipGetLastError();
+}
+template hipError_t panel_solve<double>(hipStream_t, bool, long, int, double *, long, const double *, long, const int *);
+template hipError_t panel_solve<zd>(hipStream_t, bool, long, int, zd *, long, const zd *, long, const int *);
+template hipError_t panel_solve<float>(hipStream_t, bool, long, int, float *, long, const float *, long, const int *);
+template hipError_t panel_solve<zf>(hipStream_t, bool, long, int, zf *, long, const zf *, long, const int *);
 
 // gemm<T> is this kernel for double, double complex and single complex; for
 // single data gemm<float> (gemm_lp.hip) runs its own FP32 kernel and hands

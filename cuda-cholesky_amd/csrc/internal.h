@@ -145,6 +145,13 @@ hipError_t gemm_tile(hipStream_t s, int ta, int tb, long m, long n, long k, T al
                      long lda, const T *B, long ldb, T beta, const T *C, long ldc, T *D, long ldd,
                      const GemmOpts &o = GemmOpts());
 
+// Panel solve with the inverse W = inv(L) of a diagonal block (lower triangle
+// read, ld ldw), in place, ib <= diag_max<T>() columns (rows):
+// lower: A (m x ib) <- A W^H; upper: A (ib x m) <- W A.
+template <typename T>
+hipError_t panel_solve(hipStream_t s, bool lower, long m, int ib, T *A, long lda, const T *W, long ldw,
+                       const int *abort_flag);
+
 // 2-D copy D <- S (m x n)
 template <typename T>
 hipError_t copy2d(hipStream_t s, long m, long n, const T *S, long lds, T *D, long ldd);
@@ -181,9 +188,10 @@ hipError_t herk(hipStream_t s, char uplo, char trans, long n, long k, double alp
 // ---------------------------------------------------------------------------
 template <typename T> constexpr int diag_max() { return is_complex<T>::value ? 64 : 128; }
 
-// Factor the n x n diagonal block in place (n <= diag_max<T>()), write
-// W = inv(L) densely (ld ldw) where L is the lower form of the factor
-// (L = U^H for upper), and on a non-positive pivot set *info = info_off + k + 1.
+// Factor the n x n diagonal block in place (n <= diag_max<T>()), write the
+// lower triangle of W = inv(L) (ld ldw; what is above it is unspecified) where
+// L is the lower form of the factor (L = U^H for upper), and on a non-positive
+// pivot set *info = info_off + k + 1.
 template <typename T>
 hipError_t diag_potrf(hipStream_t s, char uplo, int n, T *A, long lda, T *W, long ldw, int *info,
                       long info_off);

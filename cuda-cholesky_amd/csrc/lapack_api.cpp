@@ -75,26 +75,15 @@ hipError_t factor_panel(CULAPACKhandle h, hipStream_t s, bool lower, long n, T *
                         long j, long jb) {
   // panel slice width: one diagonal block in LDS
   constexpr int IB = hc::diag_max<T>();
-  const T one = hc::from_real<T>(1.0), mone = hc::from_real<T>(-1.0), zero = hc::from_real<T>(0.0);
+  const T one = hc::from_real<T>(1.0), mone = hc::from_real<T>(-1.0);
   auto at = [&](long r, long c) { return A + c * lda + r; };
   const char uplo = lower ? 'L' : 'U';
   for (long jj = j; jj < j + jb; jj += IB) {
     const int ib = (int)std::min<long>(IB, j + jb - jj);
     HC_TRY(hc::diag_potrf<T>(s, uplo, ib, at(jj, jj), lda, W, IB, h->dinfo, jj));
     const long r0 = jj + ib, rest = n - r0;
-    hc::GemmOpts o;
-    o.abort_flag = h->dinfo;
-    if (rest > 0) {
-      if (lower) {  // L21 <- A21 inv(L11)^H, in place: a tile spans all ib columns
-        o.min_nt = ib;
-        HC_TRY(hc::gemm<T>(s, hc::OP_N, conj_op<T>(), rest, ib, ib, one, at(r0, jj), lda, W, IB, zero,
-                           nullptr, 0, at(r0, jj), lda, o));
-      } else {      // U12 <- inv(U11^H) A12, in place: a tile spans all ib rows
-        o.min_mt = ib;
-        HC_TRY(hc::gemm<T>(s, hc::OP_N, hc::OP_N, ib, rest, ib, one, W, IB, at(jj, r0), lda, zero,
-                           nullptr, 0, at(jj, r0), lda, o));
-      }
-    }
+    // L21 <- A21 inv(L11)^H, or U12 <- inv(U11^H) A12
+    HC_TRY(hc::panel_solve<T>(s, lower, rest, ib, lower ? at(r0, jj) : at(jj, r0), lda, W, IB, h->dinfo));
     const long rem = j + jb - r0;  // panel columns still to update
     if (rem > 0) {
       hc::GemmOpts u;
