@@ -10,7 +10,7 @@
 //   diag_potrf   factor + inverse (reference lapack/dpotrf.cu:23-148 and the
 //                host dpotrf of lapack/dpotrf.c:268; here it never leaves the GPU)
 //   diag_trtri   triangular inverse (reference lapack/dtrtri.cu:23-167)
-//   diag_lauum   L^H L / U U^H      (reference lapack/dlauum.cu:23-91)
+//   diag_lauum   L^H L / U U^H      (reference lapack/dlauum.cu:23-91), single precision
 //   trsm_diag_inverses  batched inverses of op(A)'s diagonal blocks
 //   logdet       2 sum log(Re x_i)  (reference lapack/dlogdet.cu:53-118)
 #include "internal.h"
@@ -22,9 +22,6 @@
 namespace hc {
 namespace {
 
-// Factor / inverse kernels: ten waves, one per 32 x 32 (double) or 16 x 16
-// (complex) region of the lower triangle of a 4 x 4 grid of regions.
-constexpr int DIAG_THREADS = 640;
 // L^H L kernel: 512 threads in groups of TPR per row.
 constexpr int LAUUM_THREADS = 512;
 
@@ -120,20 +117,6 @@ __device__ __forceinline__ void store_lower_form(const T *S, bool lower, int n, 
   });
 }
 
-// W(r, c) = S(r, c) for r >= c, zero above; unit -> ones on the diagonal.
-// With upper, W is the conjugate transpose instead (upper triangular).
-template <typename T, int NMAX, int THREADS, typename ST = T>
-__device__ __forceinline__ void store_dense(const T *S, bool upper, int n, bool unit, ST *W, long ldw) {
-  constexpr int LS = Lds<T, NMAX>::LS;
-  for_block<NMAX, THREADS>(n, [&](int r, int c) {
-    T v = from_real<T>(0.0);
-    if (r == c) v = unit ? from_real<T>(1.0) : (upper ? conjx(S[c * LS + r]) : S[c * LS + r]);
-    else if (!upper && r > c) v = S[c * LS + r];
-    else if (upper && r < c) v = conjx(S[r * LS + c]);
-    W[(long)c * ldw + r] = convert<ST>(v);
-  });
-}
-
 // In-place R = L^H L of the lower form (lower part), columns left to right:
 // R(r, c) = sum_{k >= r} conj(L(k, r)) L(k, c).
 template <typename T, int NMAX>
@@ -153,128 +136,6 @@ __device__ __forceinline__ void lds_lauum(T *S, int n) {
     if (r < n && part == 0) S[c * LS + r] = sum;
     __syncthreads();
   }
-}
-
-// ---------------------------------------------------------------------------
-// Register-resident factor and inverse.  Each of ten waves owns one region
-// of the lower triangle (a 4 x 4 grid of NMAX/4-square regions); each lane
-// owns an RB x CB block of its wave's region in registers.  A column step
-// needs one broadcast vector, published through a double-buffered LDS array,
-// and one barrier; a wave whose region the step cannot change skips it, so
-// the work per step follows the shrinking trailing triangle.
-// ---------------------------------------------------------------------------
-template <typename T, int NMAX>
-struct Reg {
-  static constexpr int RS = NMAX / 4;          // region side (one wave)
-  static constexpr int RB = RS / 8, CB = RS / 8;  // lane block: 8 x 8 lanes per region
-  // region (I, J), I >= J, of wave w in the order (0,0) (1,0) (1,1) (2,0) ...
-  __device__ static int reg_i() {
-    const int w = threadIdx.x >> 6;
-    return w >= 6 ? 3 : (w >= 3 ? 2 : (w >= 1 ? 1 : 0));
-  }
-  __device__ static int reg_j() {
-    const int i = reg_i();
-    return (threadIdx.x >> 6) - i * (i + 1) / 2;
-  }
-  __device__ static int r0() { return reg_i() * RS + ((threadIdx.x & 63) >> 3) * RB; }
-  __device__ static int c0() { return reg_j() * RS + (threadIdx.x & 7) * CB; }
-};
-template <typename T, int NMAX>
-using RegTile = T[NMAX / 32][NMAX / 32];
-
-// Lane-wise select written per component, so a complex value never becomes
-// an aggregate select (which the compiler lowers through private memory).
-__device__ __forceinline__ double sel(bool c, double a, double b) { return c ? a : b; }
-__device__ __forceinline__ zd sel(bool c, zd a, zd b) { return make_zd(c ? a.x : b.x, c ? a.y : b.y); }
-
-// X = inv(L) of the lower form L held in LDS (S, leading dimension NMAX + 1),
-// forward substitution by rows: row k of X is final once the updates of rows
-// 0..k-1 have been applied; it is published through xrow[2][NMAX] and the
-// rows below take its contribution.  dinv[k] = 1 / L(k, k) (unused for a unit
-// diagonal).  The strict upper part of X is exactly zero throughout (it starts
-// at zero and only ever gains products with published zeros), so neither the
-// finalisation nor the update needs a column condition.  On return x holds
-// the thread's block of X.
-template <typename T, int NMAX>
-__device__ __forceinline__ void reg_trtri(const T *S, RegTile<T, NMAX> &x, T *xrow, const T *dinv, int n, bool unit) {
-  constexpr int LS = NMAX + 1, RB = Reg<T, NMAX>::RB, CB = Reg<T, NMAX>::CB;
-  const int R0 = Reg<T, NMAX>::r0(), C0 = Reg<T, NMAX>::c0();
-#pragma unroll
-  for (int ri = 0; ri < RB; ri++)
-#pragma unroll
-    for (int ci = 0; ci < CB; ci++) x[ri][ci] = from_real<T>(0.0);
-  const T one = from_real<T>(1.0), zero = from_real<T>(0.0);
-  for (int k = 0; k < n; k++) {
-    if (k >= R0 && k < R0 + RB) {  // this thread holds part of row k: finalise it
-      const T dk = unit ? one : dinv[k];
-      const int kr = k - R0;
-      T v[CB];
-#pragma unroll
-      for (int ci = 0; ci < CB; ci++) {
-        const T delta = sel(C0 + ci == k, one, zero);
-        v[ci] = zero;
-#pragma unroll
-        for (int ri = 0; ri < RB; ri++) {
-          const T fin = (delta - x[ri][ci]) * dk;
-          x[ri][ci] = sel(ri == kr, fin, x[ri][ci]);
-          v[ci] = sel(ri == kr, fin, v[ci]);
-        }
-        xrow[(k & 1) * NMAX + C0 + ci] = v[ci];
-      }
-    }
-    __syncthreads();
-    if ((Reg<T, NMAX>::reg_i() + 1) * Reg<T, NMAX>::RS > k + 1 &&
-        Reg<T, NMAX>::reg_j() * Reg<T, NMAX>::RS <= k) {  // regions with rows below k, columns <= k
-      const T *xr = xrow + (k & 1) * NMAX;
-      T lk[RB], xk[CB];
-#pragma unroll
-      for (int ri = 0; ri < RB; ri++) lk[ri] = S[k * LS + R0 + ri];
-#pragma unroll
-      for (int ci = 0; ci < CB; ci++) xk[ci] = xr[C0 + ci];
-#pragma unroll
-      for (int ri = 0; ri < RB; ri++) {
-        const bool below = R0 + ri > k;
-#pragma unroll
-        for (int ci = 0; ci < CB; ci++) {
-          const T upd = x[ri][ci] + lk[ri] * xk[ci];
-          x[ri][ci] = sel(below, upd, x[ri][ci]);
-        }
-      }
-    }
-  }
-}
-
-// Registers <-> LDS copies of the thread's block (lower part, inside n x n).
-template <typename T, int NMAX>
-__device__ __forceinline__ void reg_to_lds(const RegTile<T, NMAX> &v, T *S, int n) {
-  constexpr int LS = NMAX + 1, RB = Reg<T, NMAX>::RB, CB = Reg<T, NMAX>::CB;
-  const int R0 = Reg<T, NMAX>::r0(), C0 = Reg<T, NMAX>::c0();
-#pragma unroll
-  for (int ri = 0; ri < RB; ri++)
-#pragma unroll
-    for (int ci = 0; ci < CB; ci++) {
-      const int r = R0 + ri, c = C0 + ci;
-      if (r < n && c < n && r >= c) S[c * LS + r] = v[ri][ci];
-    }
-}
-template <typename T, int NMAX>
-__device__ __forceinline__ void lds_to_reg(const T *S, RegTile<T, NMAX> &v, int n) {
-  constexpr int LS = NMAX + 1, RB = Reg<T, NMAX>::RB, CB = Reg<T, NMAX>::CB;
-  const int R0 = Reg<T, NMAX>::r0(), C0 = Reg<T, NMAX>::c0();
-#pragma unroll
-  for (int ri = 0; ri < RB; ri++)
-#pragma unroll
-    for (int ci = 0; ci < CB; ci++) {
-      const int r = R0 + ri, c = C0 + ci;
-      v[ri][ci] = (r < n && c < n && r >= c) ? S[c * LS + r] : from_real<T>(0.0);
-    }
-}
-
-// dinv[k] = 1 / S(k, k) for k < n.
-template <typename T, int NMAX>
-__device__ __forceinline__ void diag_reciprocals(const T *S, T *dinv, int n) {
-  constexpr int LS = NMAX + 1;
-  for (int k = threadIdx.x; k < n; k += blockDim.x) dinv[k] = from_real<T>(1.0) / S[k * LS + k];
 }
 
 // ---------------------------------------------------------------------------
@@ -959,33 +820,161 @@ panel_potrf_kernel(int m, int jb, ST *A, long lda, ST *ws, int *flags, int epoch
   panel_publish(fd(b), epoch);
 }
 
+// ---------------------------------------------------------------------------
+// Triangular inverse of one block in LDS (packed lower tiles as above, lower
+// form, unit diagonals stored as ones): the 16 x 16 diagonal tiles first, one
+// wave each, then pairs of inverted blocks of w = 1, 2, 4 tiles are joined,
+// X21 = -X22 L21 X11, every tile product on the matrix cores.  T = -X22 L21 is
+// formed in registers and written over L21 before the second product, so
+// nothing but the tiles is needed.  A column-by-column substitution in
+// registers (one barrier per column) took 108 us per launch, this one 17 us
+// (128 x 128 doubles).
+// ---------------------------------------------------------------------------
+template <typename T, int NMAX>
+__device__ __forceinline__ void tiles_invert(T *S, int np) {
+  constexpr int NPMAX = NMAX / LEAF, LL = LEAF + 1, TS = LEAF * LL, NW = BLK_THREADS / 64;
+  constexpr int PER = (NPMAX * NPMAX / 4 + NW - 1) / NW;  // tiles per wave on the widest level
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto tile = [&](int I, int J) { return S + (I * (I + 1) / 2 + J) * TS; };
+  if (wave < np) {
+    T a[LEAF], x[4];
+    T *t = tile(wave, wave);
+#pragma unroll
+    for (int c = 0; c < LEAF; c++) a[c] = t[c * LL + (lane & 15)];
+    t16::leaf_inverse_cols<T>(a, x);
+#pragma unroll
+    for (int j = 0; j < 4; j++) t[((lane >> 4) + 4 * j) * LL + (lane & 15)] = x[j];
+  }
+  __syncthreads();
+  for (int w = 1; w < np; w *= 2) {
+    // tile u of the level: pair u / w^2, row and column in the pair's block 21
+    const int lw = 31 - __builtin_clz(w);
+    auto place = [&](int u, int &i, int &j, int &mid) {
+      const int base = (u >> (2 * lw)) * 2 * w;
+      mid = base + w;
+      i = mid + ((u >> lw) & (w - 1));
+      j = base + (u & (w - 1));
+      return i < np;
+    };
+    TileAcc<T> acc[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      int i, j, mid;
+      acc_zero(acc[q]);
+      if (place(wave + q * NW, i, j, mid))
+        for (int k = mid; k <= i; k++) tile_mma<false>(acc[q], tile(i, k), LL, tile(k, j), LL, -1.0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      int i, j, mid;
+      if (place(wave + q * NW, i, j, mid)) acc_store(acc[q], tile(i, j), LL);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      int i, j, mid;
+      acc_zero(acc[q]);
+      if (place(wave + q * NW, i, j, mid))
+        for (int k = j; k < mid; k++) tile_mma<false>(acc[q], tile(i, k), LL, tile(k, j), LL, 1.0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      int i, j, mid;
+      if (place(wave + q * NW, i, j, mid)) acc_store(acc[q], tile(i, j), LL);
+    }
+    __syncthreads();
+  }
+}
+
+// Packed lower tiles of the n x n block at A: lower-form element (r, c) is
+// A(r, c), or A(c, r) when swapped, conjugated when conj; identity beyond n,
+// ones on the diagonal when unit.  Lanes run along memory's contiguous index.
+template <typename T, typename ST, int NMAX>
+__device__ __forceinline__ void tiles_load(T *S, int n, const ST *A, long lda, bool swapped, bool conj, bool unit) {
+  constexpr int LL = LEAF + 1, TS = LEAF * LL, NW = BLK_THREADS / 64, NPMAX = NMAX / LEAF;
+  constexpr int PER = (NPMAX * (NPMAX + 1) / 2 + NW - 1) / NW;
+  const int lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), np = (n + LEAF - 1) / LEAF;
+  int ti[PER], tj[PER];
+  ST x[PER][4];
+#pragma unroll
+  for (int q = 0; q < PER; q++) {
+    const int t = q * NW + wave;  // row by row
+    int I = 0;
+#pragma unroll
+    for (int k = 1; k <= NPMAX; k++) I += t >= k * (k + 1) / 2 ? 1 : 0;
+    ti[q] = I < np ? I : -1;
+    tj[q] = I < np ? t - I * (I + 1) / 2 : 0;
+    const int r = max(ti[q], 0) * LEAF + (swapped ? lg : lc), c = tj[q] * LEAF + (swapped ? lc : lg);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int rr = min(swapped ? r + 4 * j : r, n - 1), cc = min(swapped ? c : c + 4 * j, n - 1);
+      x[q][j] = swapped ? A[(long)rr * lda + cc] : A[(long)cc * lda + rr];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < PER; q++) {
+    if (ti[q] < 0) continue;
+    T *t = S + (ti[q] * (ti[q] + 1) / 2 + tj[q]) * TS;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int rl = swapped ? lg + 4 * j : lc, cl = swapped ? lc : lg + 4 * j;
+      const int r = ti[q] * LEAF + rl, c = tj[q] * LEAF + cl;
+      const T v = conj ? conjx(convert<T>(x[q][j])) : convert<T>(x[q][j]);
+      const T e = t16::sel(r < n && c < n, v, from_real<T>(r == c ? 1.0 : 0.0));
+      t[cl * LL + rl] = t16::sel(unit && r == c, from_real<T>(1.0), e);
+    }
+  }
+}
+
+// fn(r, c, element) over the n x n lower-form elements r >= c held in S, or
+// with DENSE over all of them (zero above the diagonal); lanes along r, or
+// along c when swapped.
+template <typename T, int NMAX, bool DENSE, typename Fn>
+__device__ __forceinline__ void tiles_each(const T *S, int n, bool swapped, Fn fn) {
+  constexpr int LL = LEAF + 1, TS = LEAF * LL, NW = BLK_THREADS / 64;
+  const int lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), np = (n + LEAF - 1) / LEAF;
+  int t = wave + 1;
+  for (int I = 0; I < np; I++)
+    for (int J = 0; J < (DENSE ? np : I + 1); J++) {
+      if (--t != 0) continue;
+      t = NW;
+      const T *p = S + (I * (I + 1) / 2 + J) * TS;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int rl = swapped ? lg + 4 * j : lc, cl = swapped ? lc : lg + 4 * j;
+        const int r = I * LEAF + rl, c = J * LEAF + cl;
+        T v = from_real<T>(0.0);
+        if (J <= I) v = p[cl * LL + rl];
+        if (r < n && c < n && (DENSE || r >= c)) fn(r, c, v);
+      }
+    }
+}
+
 // Workgroup b inverts the diagonal block of order min(nb, ntot - b nb) at
 // (b nb, b nb) of A into the same place of B (one workgroup: nb = ntot).
-// T is the compute type, ST the storage type of A, B and W.
+// T is the compute type, ST the storage type of A and B.
 template <typename T, typename ST, int NMAX>
-__global__ void __launch_bounds__(DIAG_THREADS)
-diag_trtri_kernel(int lower, int unit, int ntot, int nb, const ST *A, long lda, ST *B, long ldb, ST *W,
-                  long ldw, const int *abort_flag) {
+__global__ void __launch_bounds__(BLK_THREADS)
+diag_trtri_kernel(int lower, int unit, int ntot, int nb, const ST *A, long lda, ST *B, long ldb,
+                  const int *abort_flag) {
   if (abort_flag != nullptr && *abort_flag != 0) return;
+  __shared__ T S[diag_lds_elems<NMAX>()];
   const long off = (long)blockIdx.x * nb;
   const int n = (int)min((long)nb, (long)ntot - off);
   A += off * lda + off;
   B += off * ldb + off;
-  constexpr int RB = Reg<T, NMAX>::RB, CB = Reg<T, NMAX>::CB;
-  __shared__ T S[NMAX * (NMAX + 1)];
-  __shared__ T vec[2 * NMAX];
-  __shared__ T dinv[NMAX];
-  load_lower_form<T, NMAX, DIAG_THREADS, ST>(S, lower, n, A, lda);
+  tiles_load<T, ST, NMAX>(S, n, A, lda, !lower, !lower, unit != 0);
   __syncthreads();
-  if (!unit) diag_reciprocals<T, NMAX>(S, dinv, n);
-  __syncthreads();
-  T x[RB][CB];
-  reg_trtri<T, NMAX>(S, x, vec, dinv, n, unit != 0);
-  __syncthreads();
-  reg_to_lds<T, NMAX>(x, S, n);
-  __syncthreads();
-  store_lower_form<T, NMAX, DIAG_THREADS, ST>(S, lower, n, B, ldb, unit != 0);
-  if (W != nullptr) store_dense<T, NMAX, DIAG_THREADS, ST>(S, false, n, unit != 0, W, ldw);
+  tiles_invert<T, NMAX>(S, (n + LEAF - 1) / LEAF);
+  tiles_each<T, NMAX, false>(S, n, !lower, [&](int r, int c, T v) {
+    if (unit && r == c) return;
+    if (lower) B[(long)c * ldb + r] = convert<ST>(v);
+    else B[(long)r * ldb + c] = convert<ST>(conjx(v));
+  });
 }
 
 // Workgroup b squares the diagonal block of order min(nb, ntot - b nb) at
@@ -993,7 +982,9 @@ diag_trtri_kernel(int lower, int unit, int ntot, int nb, const ST *A, long lda, 
 // nb = ntot, B = A, ldb = lda.
 template <typename T, typename ST, int NMAX>
 __global__ void __launch_bounds__(LAUUM_THREADS)
-diag_lauum_kernel(int lower, int ntot, int nb, const ST *A, long lda, ST *B, long ldb, long bstride) {
+diag_lauum_kernel(int lower, int ntot, int nb, const ST *A, long lda, ST *B, long ldb, long bstride,
+                  const int *abort_flag) {
+  if (abort_flag != nullptr && *abort_flag != 0) return;
   __shared__ T S[NMAX * (NMAX + 1)];
   const long off = (long)blockIdx.x * nb;
   const int n = (int)min((long)nb, (long)ntot - off);
@@ -1003,43 +994,47 @@ diag_lauum_kernel(int lower, int ntot, int nb, const ST *A, long lda, ST *B, lon
   store_lower_form<T, NMAX, LAUUM_THREADS, ST>(S, lower, n, B + blockIdx.x * bstride, ldb, false);
 }
 
-// D <- S on the triangle uplo (diagonal included) of an n x n block
+// D <- S on the triangle uplo (diagonal included) of an n x n matrix, a
+// 64 x 64 tile per workgroup
 template <typename T>
-__global__ void tri_copy_kernel(int lower, int n, const T *S, long lds, T *D, long ldd) {
-  const int r = blockIdx.x * 16 + (threadIdx.x & 15), c = blockIdx.y * 16 + (threadIdx.x >> 4);
-  if (r < n && c < n && (lower ? r >= c : r <= c)) D[(long)c * ldd + r] = S[(long)c * lds + r];
+__global__ void __launch_bounds__(256) tri_copy_kernel(int lower, int n, const T *S, long lds, T *D, long ldd,
+                                                       const int *abort_flag) {
+  if (abort_flag != nullptr && *abort_flag != 0) return;
+  const int bi = blockIdx.x, bj = blockIdx.y;
+  if (lower ? bi < bj : bi > bj) return;
+  const int r = bi * 64 + (threadIdx.x & 63), c0 = bj * 64 + (threadIdx.x >> 6);
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    T v[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = S[(long)min(c0 + 4 * (8 * h + j), n - 1) * lds + min(r, n - 1)];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const int c = c0 + 4 * (8 * h + j);
+      if (r < n && c < n && (lower ? r >= c : r <= c)) D[(long)c * ldd + r] = v[j];
+    }
+  }
 }
 
 // Block b inverts the nb x nb diagonal block of op(A) starting at b * nb.
 template <typename T, typename ST, int NMAX>
-__global__ void __launch_bounds__(DIAG_THREADS)
+__global__ void __launch_bounds__(BLK_THREADS)
 trsm_inv_kernel(int lowerlike, int op, int unit, long m, int nb, const ST *A, long lda, ST *W) {
-  constexpr int LS = Lds<T, NMAX>::LS;
-  __shared__ T S[NMAX * (NMAX + 1)];
-  __shared__ T vec[2 * NMAX];
-  __shared__ T dinv[NMAX];
+  __shared__ T S[diag_lds_elems<NMAX>()];
   const long off = (long)blockIdx.x * nb;
   const int n = (int)((m - off) < nb ? (m - off) : nb);
-  // lower form: S(r, c) = op(A)(r, c) when op(A) is lower-like, else
-  // conj(op(A)(c, r)); op(A)(i, j) = A(i, j), A(j, i) or conj(A(j, i)).
-  gather_block<NMAX, DIAG_THREADS, 16>(n, A + off * lda + off, lda, [&](int a, int b, ST x) {
-    // memory element A(off + a, off + b)
-    const T v = convert<T>(x);
-    // as an element of op(A): (a, b) for N, (b, a) for T/C
-    int r = (op == OP_N) ? a : b, c = (op == OP_N) ? b : a;
-    T e = (op == OP_C) ? conjx(v) : v;
-    if (!lowerlike) { const int t = r; r = c; c = t; e = conjx(e); }
-    if (r >= c) S[c * LS + r] = e;
+  // lower form: op(A)(r, c) when op(A) is lower-like, else conj(op(A)(c, r));
+  // op(A)(i, j) = A(i, j), A(j, i) or conj(A(j, i)).
+  const bool swapped = (op == OP_N) != (lowerlike != 0);
+  const bool conj = op == OP_N ? lowerlike == 0 : (op == OP_C) == (lowerlike != 0);
+  tiles_load<T, ST, NMAX>(S, n, A + off * lda + off, lda, swapped, conj, unit != 0);
+  __syncthreads();
+  tiles_invert<T, NMAX>(S, (n + LEAF - 1) / LEAF);
+  ST *w = W + (long)blockIdx.x * nb * nb;
+  tiles_each<T, NMAX, true>(S, n, lowerlike == 0, [&](int r, int c, T v) {
+    if (lowerlike) w[(long)c * nb + r] = convert<ST>(v);
+    else w[(long)r * nb + c] = convert<ST>(conjx(v));
   });
-  __syncthreads();
-  if (!unit) diag_reciprocals<T, NMAX>(S, dinv, n);
-  __syncthreads();
-  RegTile<T, NMAX> x;
-  reg_trtri<T, NMAX>(S, x, vec, dinv, n, unit != 0);
-  __syncthreads();
-  reg_to_lds<T, NMAX>(x, S, n);
-  __syncthreads();
-  store_dense<T, NMAX, DIAG_THREADS, ST>(S, !lowerlike, n, unit != 0, W + (long)blockIdx.x * nb * nb, nb);
 }
 
 // One workgroup scans the diagonal; info = first (upper) or last (lower)
@@ -1134,59 +1129,61 @@ hipError_t diag_potrf(hipStream_t s, char uplo, int n, ST *A, long lda, ST *W, l
 }
 
 template <typename ST>
-hipError_t diag_trtri(hipStream_t s, char uplo, char diag, int n, const ST *A, long lda, ST *B,
-                      long ldb, ST *W, long ldw, const int *abort_flag) {
+hipError_t diag_trtri(hipStream_t s, char uplo, char diag, int n, const ST *A, long lda, ST *B, long ldb,
+                      const int *abort_flag) {
   using T = typename Compute<ST>::type;
   constexpr int NMAX = diag_max<T>();
   if (n <= 0) return hipSuccess;
   if (n > NMAX) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((diag_trtri_kernel<T, ST, NMAX>), dim3(1), dim3(DIAG_THREADS), 0, s,
-                     uplo == 'L' ? 1 : 0, diag == 'U' ? 1 : 0, n, n, A, lda, B, ldb, W, ldw,
-                     abort_flag);
+  hipLaunchKernelGGL((diag_trtri_kernel<T, ST, NMAX>), dim3(1), dim3(BLK_THREADS), 0, s, uplo == 'L' ? 1 : 0,
+                     diag == 'U' ? 1 : 0, n, n, A, lda, B, ldb, abort_flag);
   return hipGetLastError();
 }
 
 template <typename ST>
-hipError_t diag_trtri_blocks(hipStream_t s, char uplo, char diag, long n, int nb, ST *A, long lda) {
+hipError_t diag_trtri_blocks(hipStream_t s, char uplo, char diag, long n, int nb, ST *A, long lda,
+                             const int *abort_flag) {
   using T = typename Compute<ST>::type;
   constexpr int NMAX = diag_max<T>();
   if (n <= 0) return hipSuccess;
   if (nb <= 0 || nb > NMAX || n > (long)INT32_MAX) return hipErrorInvalidValue;
   const long blocks = (n + nb - 1) / nb;
-  hipLaunchKernelGGL((diag_trtri_kernel<T, ST, NMAX>), dim3((unsigned)blocks), dim3(DIAG_THREADS), 0, s,
-                     uplo == 'L' ? 1 : 0, diag == 'U' ? 1 : 0, (int)n, nb, A, lda, A, lda,
-                     static_cast<ST *>(nullptr), 0L, static_cast<const int *>(nullptr));
+  hipLaunchKernelGGL((diag_trtri_kernel<T, ST, NMAX>), dim3((unsigned)blocks), dim3(BLK_THREADS), 0, s,
+                     uplo == 'L' ? 1 : 0, diag == 'U' ? 1 : 0, (int)n, nb, static_cast<const ST *>(A), lda, A, lda,
+                     abort_flag);
   return hipGetLastError();
 }
 
 template <typename ST>
-hipError_t diag_lauum(hipStream_t s, char uplo, int n, ST *A, long lda) {
+hipError_t diag_lauum(hipStream_t s, char uplo, int n, ST *A, long lda, const int *abort_flag) {
   using T = typename Compute<ST>::type;
   constexpr int NMAX = diag_max<T>();
   if (n <= 0) return hipSuccess;
   if (n > NMAX) return hipErrorInvalidValue;
   hipLaunchKernelGGL((diag_lauum_kernel<T, ST, NMAX>), dim3(1), dim3(LAUUM_THREADS), 0, s,
-                     uplo == 'L' ? 1 : 0, n, n, static_cast<const ST *>(A), lda, A, lda, 0L);
+                     uplo == 'L' ? 1 : 0, n, n, static_cast<const ST *>(A), lda, A, lda, 0L, abort_flag);
   return hipGetLastError();
 }
 
 template <typename ST>
-hipError_t diag_lauum_blocks(hipStream_t s, char uplo, long n, int nb, const ST *A, long lda, ST *W) {
+hipError_t diag_lauum_blocks(hipStream_t s, char uplo, long n, int nb, const ST *A, long lda, ST *W,
+                             const int *abort_flag) {
   using T = typename Compute<ST>::type;
   constexpr int NMAX = diag_max<T>();
   if (n <= 0) return hipSuccess;
   if (nb <= 0 || nb > NMAX || n > (long)INT32_MAX) return hipErrorInvalidValue;
   const long blocks = (n + nb - 1) / nb;
   hipLaunchKernelGGL((diag_lauum_kernel<T, ST, NMAX>), dim3((unsigned)blocks), dim3(LAUUM_THREADS), 0, s,
-                     uplo == 'L' ? 1 : 0, (int)n, nb, A, lda, W, (long)nb, (long)nb * nb);
+                     uplo == 'L' ? 1 : 0, (int)n, nb, A, lda, W, (long)nb, (long)nb * nb, abort_flag);
   return hipGetLastError();
 }
 
 template <typename T>
-hipError_t tri_copy(hipStream_t s, char uplo, int n, const T *S, long lds, T *D, long ldd) {
+hipError_t tri_copy(hipStream_t s, char uplo, long n, const T *S, long lds, T *D, long ldd, const int *abort_flag) {
   if (n <= 0) return hipSuccess;
-  const dim3 grid((unsigned)((n + 15) / 16), (unsigned)((n + 15) / 16));
-  hipLaunchKernelGGL((tri_copy_kernel<T>), grid, dim3(256), 0, s, uplo == 'L' ? 1 : 0, n, S, lds, D, ldd);
+  const unsigned t = (unsigned)((n + 63) / 64);
+  hipLaunchKernelGGL((tri_copy_kernel<T>), dim3(t, t), dim3(256), 0, s, uplo == 'L' ? 1 : 0, (int)n, S, lds, D, ldd,
+                     abort_flag);
   return hipGetLastError();
 }
 
@@ -1200,7 +1197,7 @@ hipError_t trsm_diag_inverses(hipStream_t s, char uplo, char trans, char diag, l
   const int op = is_complex<T>::value ? op_code(trans) : (trans == 'N' ? OP_N : OP_T);
   const int lowerlike = ((uplo == 'L') == (trans == 'N')) ? 1 : 0;
   const unsigned nblk = (unsigned)((m + nb - 1) / nb);
-  hipLaunchKernelGGL((trsm_inv_kernel<T, ST, NMAX>), dim3(nblk), dim3(DIAG_THREADS), 0, s, lowerlike,
+  hipLaunchKernelGGL((trsm_inv_kernel<T, ST, NMAX>), dim3(nblk), dim3(BLK_THREADS), 0, s, lowerlike,
                      op, diag == 'U' ? 1 : 0, m, nb, A, lda, W);
   return hipGetLastError();
 }
@@ -1241,11 +1238,11 @@ template hipError_t panel_potrf<double>(hipStream_t, long, long, double *, long,
 #define HC_INST(T)                                                                            \
   template hipError_t diag_potrf<T>(hipStream_t, char, int, T *, long, T *, long, int *, long); \
   template hipError_t diag_trtri<T>(hipStream_t, char, char, int, const T *, long, T *, long,   \
-                                    T *, long, const int *);                                    \
-  template hipError_t diag_trtri_blocks<T>(hipStream_t, char, char, long, int, T *, long);      \
-  template hipError_t diag_lauum<T>(hipStream_t, char, int, T *, long);                         \
-  template hipError_t diag_lauum_blocks<T>(hipStream_t, char, long, int, const T *, long, T *); \
-  template hipError_t tri_copy<T>(hipStream_t, char, int, const T *, long, T *, long);          \
+                                    const int *);                                               \
+  template hipError_t diag_trtri_blocks<T>(hipStream_t, char, char, long, int, T *, long,       \
+                                           const int *);                                        \
+  template hipError_t tri_copy<T>(hipStream_t, char, long, const T *, long, T *, long,          \
+                                  const int *);                                                 \
   template hipError_t trsm_diag_inverses<T>(hipStream_t, char, char, char, long, int,           \
                                             const T *, long, T *);                              \
   template hipError_t diag_zero_scan<T>(hipStream_t, char, long, const T *, long, int *);       \
@@ -1258,5 +1255,12 @@ HC_INST(zd)
 HC_INST(float)
 HC_INST(zf)
 #undef HC_INST
+// squares of single-precision diagonal blocks (formed in double)
+#define HC_INST_SQ(T)                                                                              \
+  template hipError_t diag_lauum<T>(hipStream_t, char, int, T *, long, const int *);               \
+  template hipError_t diag_lauum_blocks<T>(hipStream_t, char, long, int, const T *, long, T *, const int *);
+HC_INST_SQ(float)
+HC_INST_SQ(zf)
+#undef HC_INST_SQ
 
 }  // namespace hc

@@ -22,6 +22,8 @@
 // epilogue writes 128-byte column segments (coalesced).
 // Complex products use four real MFMAs (re*re - im*im, re*im + im*re) on
 // separate real / imaginary LDS planes.
+#include <algorithm>
+
 #include "internal.h"
 
 namespace hc {
@@ -89,6 +91,10 @@ struct KParams {
   // tri-grid launches: the number of tiles when the grid is smaller (each
   // workgroup then takes tiles w, w + gridDim.x, ...); 0: one per tile
   int vtiles;
+  // batch > 0: product z = blockIdx.z of the batch at A + z bsA, B + z bsB,
+  // D + z bsD, the last one of size last_m x last_n x last_k (beta = 0)
+  int batch, last_m, last_n, last_k;
+  long bsA, bsB, bsD;
 };
 
 // Element (r, c) of op(X).
@@ -151,6 +157,15 @@ __device__ __forceinline__ int xcd_contiguous(int w, int nwg) {
   return x < rem ? x * (base + 1) + i : rem * (base + 1) + (x - rem) * base + i;
 }
 
+// Logical index of workgroup w of nwg with chunks of 32 logical tiles dealt
+// round-robin to the XCDs (the remainder that is no whole round as it comes).
+__device__ __forceinline__ int xcd_chunked(int w, int nwg) {
+  constexpr int CH = 32;
+  if (w >= nwg / (NXCD * CH) * (NXCD * CH)) return w;
+  const int x = w % NXCD, i = w / NXCD;
+  return (i / CH * NXCD + x) * CH + i % CH;
+}
+
 // Position i of the order n - 1, 0, n - 2, 1, ... (high_first) or
 // 0, n - 1, 1, n - 2, ...: a permutation of [0, n).
 __device__ __forceinline__ int serpentine(int i, int n, bool high_first) {
@@ -161,6 +176,19 @@ __device__ __forceinline__ int serpentine(int i, int n, bool high_first) {
 template <typename T, int TA, int TB, int MT, int NT, bool TG>
 __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
   if (p.abort_flag != nullptr && *p.abort_flag != 0) return;
+  if constexpr (!TG) {
+    if (p.batch > 0) {
+      const int z = (int)blockIdx.z;
+      p.A += z * p.bsA;
+      p.B += z * p.bsB;
+      p.D += z * p.bsD;
+      if (z == p.batch - 1) {
+        p.m = p.last_m;
+        p.n = p.last_n;
+        p.k = p.last_k;
+      }
+    }
+  }
 
   constexpr bool CPLX = is_complex<T>::value;
   using R = typename Prec<T>::R;
@@ -186,7 +214,11 @@ __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
   // walk tiles in groups of GROUP tile rows, column by column inside a group,
   // so the tiles in flight on one XCD share their op(A) and op(B) panels.
   auto tile_body = [&](const int wid, const int nwg) __attribute__((always_inline)) {
-  const int logical = xcd_contiguous(wid, nwg);
+  // A triangular product over a triangular grid (L^H L): a tile's K range
+  // shrinks along the logical order, so contiguous ranges would leave the
+  // XCDs with unequal work: chunks of the order are dealt in turn (heaviest
+  // tiles first everywhere).
+  const int logical = TG && p.tri_a != TRI_NONE ? xcd_chunked(wid, nwg) : xcd_contiguous(wid, nwg);
   int bm, bn;
   if constexpr (TG) {
     // row-major position of the logical tile in the lower triangle of tiles
@@ -234,6 +266,9 @@ __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
     if (p.tri_b != TRI_NONE && p.tri_b == TRI_UPPER) bn = gy - 1 - bn;
   }
   const int m0 = bm * MT, n0 = bn * NT;
+  if constexpr (!TG) {
+    if (p.batch > 0 && (m0 >= p.m || n0 >= p.n)) return;  // the last product may be smaller
+  }
 
   // ---- K range: a triangular operand bounds it ----
   int kbeg = 0, kend = p.k;
@@ -524,7 +559,8 @@ hipError_t launch(hipStream_t s, const KParams<T> &p) {
                        p.ldc, p.D, p.ldd);
     return hipGetLastError();
   }
-  const dim3 grid((unsigned)((p.m + MT - 1) / MT), (unsigned)((p.n + NT - 1) / NT));
+  const dim3 grid((unsigned)((p.m + MT - 1) / MT), (unsigned)((p.n + NT - 1) / NT),
+                  (unsigned)(p.batch > 0 ? p.batch : 1));
   hipLaunchKernelGGL((gemm_kernel<T, TA, TB, MT, NT, false>), grid, dim3(NTHREADS), 0, s, p);
   return hipGetLastError();
 }
@@ -731,7 +767,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) panel_solve_kernel(long m, int ib
 }
 
 template <typename T>
-__global__ void copy2d_kernel(int m, int n, const T *S, long lds, T *D, long ldd) {
+__global__ void copy2d_kernel(int m, int n, const T *S, long lds, T *D, long ldd, const int *abort_flag) {
+  if (abort_flag != nullptr && *abort_flag != 0) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int j = blockIdx.y;
   if (i < m && j < n) D[(long)j * ldd + i] = S[(long)j * lds + i];
@@ -756,6 +793,10 @@ hipError_t gemm_tile(hipStream_t s, int ta, int tb, long m, long n, long k, T al
   p.kchunk = 0;
   p.part = nullptr;
   p.vtiles = 0;
+  p.batch = o.batch;
+  p.last_m = (int)o.last_m; p.last_n = (int)o.last_n; p.last_k = (int)o.last_k;
+  p.bsA = o.bsA; p.bsB = o.bsB; p.bsD = o.bsD;
+  if (o.batch > 0 && (o.tri_grid || o.splitk_ws != nullptr || !is_zero(beta))) return hipErrorInvalidValue;
 
   // Tile choice: the large tile when the launch has at least the measured
   // number of them (family D / Z of the tuning table; about one workgroup per
@@ -764,7 +805,7 @@ hipError_t gemm_tile(hipStream_t s, int ta, int tb, long m, long n, long k, T al
   constexpr bool CPLX = is_complex<T>::value;
   constexpr int BIG = CPLX ? 64 : 128, SMALL = CPLX ? 32 : 64;
   const long tb_m = (m + BIG - 1) / BIG, tb_n = (n + BIG - 1) / BIG;
-  const long tiles_big = o.tri_grid ? tb_m * (tb_m + 1) / 2 : tb_m * tb_n;
+  const long tiles_big = (o.tri_grid ? tb_m * (tb_m + 1) / 2 : tb_m * tb_n) * std::max(o.batch, 1);
   int mt = tiles_big >= tuned_tile_min(CPLX ? 'Z' : 'D', 240) ? BIG : SMALL, nt = mt;
   // real data with at most 16 columns and plenty of row tiles: 128 x 16 tiles
   if (!CPLX && tb == OP_N && n <= 16 && o.tri_b == TRI_NONE && o.min_nt <= 16 && !o.tri_grid &&
@@ -796,10 +837,10 @@ hipError_t gemm_tile(hipStream_t s, int ta, int tb, long m, long n, long k, T al
 }
 
 template <typename T>
-hipError_t copy2d(hipStream_t s, long m, long n, const T *S, long lds, T *D, long ldd) {
+hipError_t copy2d(hipStream_t s, long m, long n, const T *S, long lds, T *D, long ldd, const int *abort_flag) {
   if (m <= 0 || n <= 0) return hipSuccess;
   dim3 grid((unsigned)((m + 255) / 256), (unsigned)n);
-  hipLaunchKernelGGL((copy2d_kernel<T>), grid, dim3(256), 0, s, (int)m, (int)n, S, lds, D, ldd);
+  hipLaunchKernelGGL((copy2d_kernel<T>), grid, dim3(256), 0, s, (int)m, (int)n, S, lds, D, ldd, abort_flag);
   return hipGetLastError();
 }
 
@@ -846,11 +887,14 @@ hipError_t gemm(hipStream_t s, int ta, int tb, long m, long n, long k, T alpha, 
 HC_GEMM_INST(gemm, double)
 HC_GEMM_INST(gemm, zd)
 HC_GEMM_INST(gemm, zf)
+HC_GEMM_INST(gemm_tile, double)
+HC_GEMM_INST(gemm_tile, zd)
 HC_GEMM_INST(gemm_tile, float)
+HC_GEMM_INST(gemm_tile, zf)
 #undef HC_GEMM_INST
-template hipError_t copy2d<double>(hipStream_t, long, long, const double *, long, double *, long);
-template hipError_t copy2d<zd>(hipStream_t, long, long, const zd *, long, zd *, long);
-template hipError_t copy2d<float>(hipStream_t, long, long, const float *, long, float *, long);
-template hipError_t copy2d<zf>(hipStream_t, long, long, const zf *, long, zf *, long);
+template hipError_t copy2d<double>(hipStream_t, long, long, const double *, long, double *, long, const int *);
+template hipError_t copy2d<zd>(hipStream_t, long, long, const zd *, long, zd *, long, const int *);
+template hipError_t copy2d<float>(hipStream_t, long, long, const float *, long, float *, long, const int *);
+template hipError_t copy2d<zf>(hipStream_t, long, long, const zf *, long, zf *, long, const int *);
 
 }  // namespace hc

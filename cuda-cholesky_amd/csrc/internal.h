@@ -126,6 +126,11 @@ struct GemmOpts {
   void *splitk_ws = nullptr;  // optional workspace: few-column products may split K
   long splitk_elems = 0;      // ... of this many elements
   int max_wgs = 0;            // tri_grid: at most this many workgroups (0: one per tile)
+  // gemm_tile only, beta = 0: batch products of the same size (the last one
+  // last_m x last_n x last_k, no larger) at strides of bsA, bsB, bsD elements
+  int batch = 0;
+  long last_m = 0, last_n = 0, last_k = 0;
+  long bsA = 0, bsB = 0, bsD = 0;
 };
 
 template <typename T>
@@ -154,7 +159,8 @@ hipError_t panel_solve(hipStream_t s, bool lower, long m, int ib, T *A, long lda
 
 // 2-D copy D <- S (m x n)
 template <typename T>
-hipError_t copy2d(hipStream_t s, long m, long n, const T *S, long lds, T *D, long ldd);
+hipError_t copy2d(hipStream_t s, long m, long n, const T *S, long lds, T *D, long ldd,
+                  const int *abort_flag = nullptr);
 
 
 // ---------------------------------------------------------------------------
@@ -208,25 +214,28 @@ inline long panel_ws_elems(long jb) { return 2 * ((jb + 127) / 128) * 128L * 128
 template <typename T>
 hipError_t panel_potrf(hipStream_t s, long m, long jb, T *A, long lda, T *ws, int *flags, int epoch, int *info,
                        long info_off);
-// Invert the triangular block in place (B = inv(A), B may equal A) and, when
-// W != nullptr, also write inv of its lower form densely into W.
+// B = inv(A) of a triangular block of order n <= diag_max<T>() (B may equal A).
 template <typename T>
-hipError_t diag_trtri(hipStream_t s, char uplo, char diag, int n, const T *A, long lda, T *B,
-                      long ldb, T *W, long ldw, const int *abort_flag);
+hipError_t diag_trtri(hipStream_t s, char uplo, char diag, int n, const T *A, long lda, T *B, long ldb,
+                      const int *abort_flag);
 // Every nb x nb diagonal block of the n x n triangle inverted in place, one
 // workgroup each (the last block may be smaller).
 template <typename T>
-hipError_t diag_trtri_blocks(hipStream_t s, char uplo, char diag, long n, int nb, T *A, long lda);
-// U U^H / L^H L of every nb x nb diagonal block of the n x n triangle, block
-// b into W + b nb^2 (ld nb, triangle uplo only), one workgroup each.
+hipError_t diag_trtri_blocks(hipStream_t s, char uplo, char diag, long n, int nb, T *A, long lda,
+                             const int *abort_flag);
+// D <- S on the triangle uplo (diagonal included) of an n x n matrix.
 template <typename T>
-hipError_t diag_lauum_blocks(hipStream_t s, char uplo, long n, int nb, const T *A, long lda, T *W);
-// D <- S on the triangle uplo (diagonal included) of an n x n block.
+hipError_t tri_copy(hipStream_t s, char uplo, long n, const T *S, long lds, T *D, long ldd,
+                    const int *abort_flag);
+// In-place U U^H (upper) or L^H L (lower) of a single-precision diagonal block
+// (float, zf), formed in double.
 template <typename T>
-hipError_t tri_copy(hipStream_t s, char uplo, int n, const T *S, long lds, T *D, long ldd);
-// In-place U U^H (upper) or L^H L (lower) of a diagonal block.
+hipError_t diag_lauum(hipStream_t s, char uplo, int n, T *A, long lda, const int *abort_flag);
+// The same of every nb x nb diagonal block of the n x n triangle, block b into
+// W + b nb^2 (ld nb, triangle uplo only), one workgroup each.
 template <typename T>
-hipError_t diag_lauum(hipStream_t s, char uplo, int n, T *A, long lda);
+hipError_t diag_lauum_blocks(hipStream_t s, char uplo, long n, int nb, const T *A, long lda, T *W,
+                             const int *abort_flag);
 // Batched inverses of the nb x nb diagonal blocks of op(A) (order m) into W,
 // block b at W + b * nb * nb with leading dimension nb.
 template <typename T>

@@ -320,69 +320,142 @@ hipError_t potrf_device(CULAPACKhandle h, char uplo, long n, T *A, long lda, T *
   return hipSuccess;
 }
 
-// Recursive triangular inverse: inv([A11 0; A21 A22]) =
-// [X11 0; -X22 A21 X11  X22] (lower; upper is the mirror).  The reference's
-// loop (lapack/dtrtri.c:360-458) walks nb-column blocks; halving instead keeps
-// the two TRMMs per level large.  X holds an n2 x n1 intermediate.
-// The leaves (IB x IB diagonal blocks at multiples of IB: every split point
-// is one) only read their own block, which no product of the recursion
-// writes, so they are all inverted first, in one launch.
+// Triangular inverse by levels: the IB x IB diagonal blocks are inverted in one
+// launch, then at each level b = IB, 2 IB, ... every pair of neighbouring
+// inverted blocks is joined, inv([A11 0; A21 A22]) = [X11 0; -X22 A21 X11  X22]
+// (lower; upper is the mirror), all pairs of a level in one batched launch per
+// product.  The reference's loop (lapack/dtrtri.c:360-458) walks nb-column
+// blocks.  The same products in recursive order are two launches per pair: at
+// n = 6001, 94 launches of 20 us or more each against 12 (the level products
+// are the recursion's, with the same number of operations).  X: workspace of
+// trtri_ws_elems elements for the intermediates -X22 A21.
 template <typename T>
-hipError_t trtri_rec(hipStream_t s, char uplo, char diag, long n, T *A, long lda, T *X, bool top = true) {
-  constexpr int IB = hc::diag_max<T>();
-  if (n <= IB) return top ? hc::diag_trtri<T>(s, uplo, diag, (int)n, A, lda, A, lda, nullptr, 0, nullptr)
-                          : hipSuccess;
-  if (top) HC_TRY(hc::diag_trtri_blocks<T>(s, uplo, diag, n, IB, A, lda));
-  const long n1 = ((n / 2 + IB - 1) / IB) * IB, n2 = n - n1;
-  T *A11 = A, *A22 = A + n1 * lda + n1;
-  HC_TRY(trtri_rec(s, uplo, diag, n1, A11, lda, X, false));
-  HC_TRY(trtri_rec(s, uplo, diag, n2, A22, lda, X, false));
-  const T one = hc::from_real<T>(1.0), mone = hc::from_real<T>(-1.0);
-  if (uplo == 'L') {
-    T *A21 = A + n1;
-    HC_TRY(hc::trmm<T>(s, 'L', 'L', 'N', diag, n2, n1, mone, A22, lda, A21, lda, X, n2));
-    return hc::trmm<T>(s, 'R', 'L', 'N', diag, n2, n1, one, A11, lda, X, n2, A21, lda);
+size_t trtri_ws_elems(long n) {
+  size_t most = 0;
+  for (long b = hc::diag_max<T>(); b < n; b *= 2) {
+    const long pairs = (n - b + 2 * b - 1) / (2 * b);
+    // one b x b intermediate per pair; a single pair's is only as large as its product
+    most = std::max(most, pairs > 1 ? (size_t)pairs * b * b : (size_t)b * std::min(b, n - b));
   }
-  T *A12 = A + n1 * lda;
-  HC_TRY(hc::trmm<T>(s, 'L', 'U', 'N', diag, n1, n2, mone, A11, lda, A12, lda, X, n1));
-  return hc::trmm<T>(s, 'R', 'U', 'N', diag, n1, n2, one, A22, lda, X, n1, A12, lda);
+  return most;
 }
 
-// Recursive triangular square: lower L^H L =
-// [L11^H L11 + L21^H L21, .; L22^H L21, L22^H L22]; upper U U^H mirrors it.
-// The reference's loop is lapack/dlauum.c:188-281.
-// A leaf (IB x IB diagonal block at a multiple of IB) still holds its factor
-// block when the recursion reaches it, but the products above it read that
-// block until then, so the leaves are squared beforehand into `leaves`
-// (block b at leaves + b IB^2, one launch) and only copied into place here.
 template <typename T>
-hipError_t lauum_rec(hipStream_t s, char uplo, long n, T *A, long lda, T *X, const T *leaves) {
+hipError_t trtri_device(hipStream_t s, char uplo, char diag, long n, T *A, long lda, T *X, const int *abort_flag) {
   constexpr int IB = hc::diag_max<T>();
-  if (n <= IB) return hc::tri_copy<T>(s, uplo, (int)n, leaves, IB, A, lda);
-  const long n1 = ((n / 2 + IB - 1) / IB) * IB, n2 = n - n1;
+  HC_TRY(hc::diag_trtri_blocks<T>(s, uplo, diag, n, IB, A, lda, abort_flag));
+  const T one = hc::from_real<T>(1.0), mone = hc::from_real<T>(-1.0), zero = hc::from_real<T>(0.0);
+  const bool lower = uplo == 'L';
+  for (long b = IB; b < n; b *= 2) {
+    const long pairs = (n - b + 2 * b - 1) / (2 * b), last = std::min(b, n - (2 * pairs - 1) * b);
+    const long step = 2 * b * (lda + 1), ldx = lower && pairs == 1 ? last : b;
+    T *A11 = A, *A22 = A + b * (lda + 1), *Aod = lower ? A + b : A + b * lda;
+    hc::GemmOpts o;
+    o.abort_flag = abort_flag;
+    o.unit = diag == 'U';
+    o.batch = (int)pairs;
+    // -X22 A21 (lower, the last pair's 22 block may be smaller), -X11 A12 (upper)
+    hc::GemmOpts p = o;
+    p.tri_a = lower ? hc::TRI_LOWER : hc::TRI_UPPER;
+    p.bsA = p.bsB = step;
+    p.bsD = b * b;
+    p.last_m = lower ? last : b;
+    p.last_n = lower ? b : last;
+    p.last_k = lower ? last : b;
+    HC_TRY(hc::gemm_tile<T>(s, hc::OP_N, hc::OP_N, b, b, b, mone, lower ? A22 : A11, lda, Aod, lda, zero, nullptr, 0,
+                            X, ldx, p));
+    // times X11 (lower), X22 (upper)
+    p = o;
+    p.tri_b = lower ? hc::TRI_LOWER : hc::TRI_UPPER;
+    p.bsA = b * b;
+    p.bsB = p.bsD = step;
+    p.last_m = lower ? last : b;
+    p.last_n = lower ? b : last;
+    p.last_k = lower ? b : last;
+    HC_TRY(hc::gemm_tile<T>(s, hc::OP_N, hc::OP_N, b, b, b, one, X, ldx, lower ? A11 : A22, lda, zero, nullptr, 0, Aod,
+                            lda, p));
+  }
+  return hipSuccess;
+}
+
+// Triangular square, lower L^H L, upper U U^H (the reference's loop is
+// lapack/dlauum.c:188-281).  Double and double complex up to order kSquareMax:
+// one product over the tiles of the result's triangle, with K cut to the rows
+// below both tiles, into the workspace, and a copy of the triangle.  Above, and
+// for single precision: [L11^H L11 + L21^H L21, .; L22^H L21, L22^H L22]
+// recursively (upper mirrors it), which keeps the workspace at a quarter of the
+// matrix.  Recursing down to the diagonal blocks is three launches per pair of
+// them; single precision keeps it because its diagonal blocks are squared in
+// double (leaves: beforehand, in one launch, since the products above a block
+// still read its factor; block b at leaves + b IB^2).
+constexpr long kSquareMax = 8192;
+
+template <typename T> constexpr bool is_single() { return std::is_same<T, float>::value || std::is_same<T, hc::zf>::value; }
+
+template <typename T>
+size_t lauum_rec_elems(long n) {
+  constexpr int IB = hc::diag_max<T>();
+  const long leaf = is_single<T>() ? IB : kSquareMax;
+  if (n <= leaf) return is_single<T>() ? 0 : (size_t)n * (size_t)n;
+  const long n1 = (n / 2 + IB - 1) / IB * IB;
+  return std::max({(size_t)n1 * (size_t)(n - n1), lauum_rec_elems<T>(n1), lauum_rec_elems<T>(n - n1)});
+}
+template <typename T>
+size_t lauum_ws_elems(long n) {
+  constexpr int IB = hc::diag_max<T>();
+  const size_t leaves = is_single<T>() && n > IB ? (size_t)((n + IB - 1) / IB) * IB * IB : 0;
+  return lauum_rec_elems<T>(n) + leaves;
+}
+
+template <typename T>
+hipError_t lauum_rec(hipStream_t s, char uplo, long n, T *A, long lda, T *X, const T *leaves, const int *abort_flag) {
+  constexpr int IB = hc::diag_max<T>();
+  const T one = hc::from_real<T>(1.0), zero = hc::from_real<T>(0.0);
+  const bool lower = uplo == 'L';
+  hc::GemmOpts o;
+  o.abort_flag = abort_flag;
+  if (is_single<T>()) {
+    if (n <= IB) return hc::tri_copy<T>(s, uplo, n, leaves, IB, A, lda, abort_flag);
+  } else if (n <= kSquareMax) {
+    o.tri_grid = true;
+    o.real_diag = hc::is_complex<T>::value;
+    o.tri_out = lower ? hc::TRI_LOWER : hc::TRI_UPPER;
+    o.tri_a = hc::TRI_UPPER;  // L^H, U
+    o.tri_b = hc::TRI_LOWER;  // L, U^H
+    HC_TRY(hc::gemm_tile<T>(s, lower ? conj_op<T>() : hc::OP_N, lower ? hc::OP_N : conj_op<T>(), n, n, n, one, A, lda,
+                            A, lda, zero, nullptr, 0, X, n, o));
+    return hc::tri_copy<T>(s, uplo, n, X, n, A, lda, abort_flag);
+  }
+  const long n1 = (n / 2 + IB - 1) / IB * IB, n2 = n - n1;
   T *A11 = A, *A22 = A + n1 * lda + n1;
-  const T one = hc::from_real<T>(1.0);
-  HC_TRY(lauum_rec(s, uplo, n1, A11, lda, X, leaves));
-  if (uplo == 'L') {
+  HC_TRY(lauum_rec(s, uplo, n1, A11, lda, X, leaves, abort_flag));
+  if (lower) {
     T *A21 = A + n1;
-    HC_TRY(hc::herk<T>(s, 'L', 'C', n1, n2, 1.0, A21, lda, 1.0, A11, lda));
-    HC_TRY(hc::trmm<T>(s, 'L', 'L', 'C', 'N', n2, n1, one, A22, lda, A21, lda, X, n2));
-    HC_TRY(hc::copy2d<T>(s, n2, n1, X, n2, A21, lda));
+    HC_TRY(hc::herk<T>(s, 'L', 'C', n1, n2, 1.0, A21, lda, 1.0, A11, lda, abort_flag));
+    o.tri_a = hc::TRI_UPPER;
+    HC_TRY(hc::gemm_tile<T>(s, conj_op<T>(), hc::OP_N, n2, n1, n2, one, A22, lda, A21, lda, zero, nullptr, 0, X, n2, o));
+    HC_TRY(hc::copy2d<T>(s, n2, n1, X, n2, A21, lda, abort_flag));
   } else {
     T *A12 = A + n1 * lda;
-    HC_TRY(hc::herk<T>(s, 'U', 'N', n1, n2, 1.0, A12, lda, 1.0, A11, lda));
-    HC_TRY(hc::trmm<T>(s, 'R', 'U', 'C', 'N', n1, n2, one, A22, lda, A12, lda, X, n1));
-    HC_TRY(hc::copy2d<T>(s, n1, n2, X, n1, A12, lda));
+    HC_TRY(hc::herk<T>(s, 'U', 'N', n1, n2, 1.0, A12, lda, 1.0, A11, lda, abort_flag));
+    o.tri_b = hc::TRI_LOWER;
+    HC_TRY(hc::gemm_tile<T>(s, hc::OP_N, conj_op<T>(), n1, n2, n2, one, A12, lda, A22, lda, zero, nullptr, 0, X, n1, o));
+    HC_TRY(hc::copy2d<T>(s, n1, n2, X, n1, A12, lda, abort_flag));
   }
-  return lauum_rec(s, uplo, n2, A22, lda, X, leaves + (n1 / IB) * (long)IB * IB);
+  return lauum_rec(s, uplo, n2, A22, lda, X, leaves == nullptr ? nullptr : leaves + (n1 / IB) * (long)IB * IB,
+                   abort_flag);
 }
 
 template <typename T>
-size_t rec_ws_bytes(long n) {
-  constexpr int IB = hc::diag_max<T>();
-  if (n <= IB) return 0;
-  const long n1 = ((n / 2 + IB - 1) / IB) * IB;
-  return (size_t)n1 * (size_t)(n - n1) * sizeof(T);
+hipError_t lauum_device(hipStream_t s, char uplo, long n, T *A, long lda, T *X, const int *abort_flag) {
+  T *leaves = nullptr;
+  if constexpr (is_single<T>()) {
+    constexpr int IB = hc::diag_max<T>();
+    if (n <= IB) return hc::diag_lauum<T>(s, uplo, (int)n, A, lda, abort_flag);
+    leaves = X + lauum_rec_elems<T>(n);
+    HC_TRY(hc::diag_lauum_blocks<T>(s, uplo, n, IB, A, lda, leaves, abort_flag));
+  }
+  return lauum_rec<T>(s, uplo, n, A, lda, X, leaves, abort_flag);
 }
 
 // Copies the device info word back and waits for the handle's streams.
@@ -416,6 +489,27 @@ CUresult potrf_api(const char *name, CULAPACKhandle h, CBlasUplo uplo, size_t n,
   return finish(h, info);
 }
 
+// TRTRI and / or LAUUM of the n x n triangle at A.  A non-unit triangle to be
+// inverted is first scanned for zeros on its diagonal into the info word, which
+// every kernel behind it reads: a singular one stays unchanged, and the host
+// waits once, at the end.
+template <typename T>
+CUresult triangle_ops(CULAPACKhandle h, CBlasUplo uplo, CBlasDiag diag, size_t n, T *A, size_t lda, bool invert,
+                      bool square, long *info) {
+  const size_t elems = std::max(invert ? trtri_ws_elems<T>((long)n) : 0, square ? lauum_ws_elems<T>((long)n) : 0);
+  void *ws = nullptr;
+  HC_CHECK(workspace(h, elems * sizeof(T) + 256, &ws));
+  const bool scan = invert && diag == CBlasNonUnit;
+  const int *flag = scan ? h->dinfo : nullptr;
+  if (scan) HC_CHECK(hc::diag_zero_scan<T>(h->stream, (char)uplo, (long)n, A, (long)lda, h->dinfo));
+  if (invert)
+    HC_CHECK(trtri_device<T>(h->stream, (char)uplo, (char)diag, (long)n, A, (long)lda, static_cast<T *>(ws), flag));
+  if (square) HC_CHECK(lauum_device<T>(h->stream, (char)uplo, (long)n, A, (long)lda, static_cast<T *>(ws), flag));
+  if (scan) return finish(h, info);
+  HC_CHECK(hipStreamSynchronize(h->stream));
+  return CUDA_SUCCESS;
+}
+
 template <typename T>
 CUresult trtri_api(const char *name, CULAPACKhandle h, CBlasUplo uplo, CBlasDiag diag, size_t n,
                    CUdeviceptr A, size_t lda, long *info) {
@@ -429,17 +523,7 @@ CUresult trtri_api(const char *name, CULAPACKhandle h, CBlasUplo uplo, CBlasDiag
   if (n == 0) return CUDA_SUCCESS;
   hc::DeviceGuard g(h->device);
   HC_CHECK(g.status());
-  T *Ap = dptr<T>(A);
-  if (diag == CBlasNonUnit) {
-    HC_CHECK(hc::diag_zero_scan<T>(h->stream, (char)uplo, (long)n, Ap, (long)lda, h->dinfo));
-    CUresult r = finish(h, info);
-    if (r != CUDA_SUCCESS || *info != 0) return r;
-  }
-  void *ws = nullptr;
-  HC_CHECK(workspace(h, rec_ws_bytes<T>((long)n) + 256, &ws));
-  HC_CHECK(trtri_rec<T>(h->stream, (char)uplo, (char)diag, (long)n, Ap, (long)lda, static_cast<T *>(ws)));
-  HC_CHECK(hipStreamSynchronize(h->stream));
-  return CUDA_SUCCESS;
+  return triangle_ops<T>(h, uplo, diag, n, dptr<T>(A), lda, true, false, info);
 }
 
 template <typename T>
@@ -454,20 +538,7 @@ CUresult lauum_api(const char *name, CULAPACKhandle h, CBlasUplo uplo, size_t n,
   if (n == 0) return CUDA_SUCCESS;
   hc::DeviceGuard g(h->device);
   HC_CHECK(g.status());
-  void *ws = nullptr;
-  constexpr int IB = hc::diag_max<T>();
-  if ((long)n <= IB) {
-    HC_CHECK(hc::diag_lauum<T>(h->stream, (char)uplo, (int)n, dptr<T>(A), (long)lda));
-  } else {
-    const size_t xb = (rec_ws_bytes<T>((long)n) + 255) / 256 * 256;
-    const size_t lb = (size_t)((n + IB - 1) / IB) * IB * IB * sizeof(T);
-    HC_CHECK(workspace(h, xb + lb, &ws));
-    T *leaves = reinterpret_cast<T *>(static_cast<char *>(ws) + xb);
-    HC_CHECK(hc::diag_lauum_blocks<T>(h->stream, (char)uplo, (long)n, IB, dptr<const T>(A), (long)lda, leaves));
-    HC_CHECK(lauum_rec<T>(h->stream, (char)uplo, (long)n, dptr<T>(A), (long)lda, static_cast<T *>(ws), leaves));
-  }
-  HC_CHECK(hipStreamSynchronize(h->stream));
-  return CUDA_SUCCESS;
+  return triangle_ops<T>(h, uplo, CBlasNonUnit, n, dptr<T>(A), lda, false, true, info);
 }
 
 template <typename T>
@@ -480,9 +551,9 @@ CUresult potri_api(const char *name, CULAPACKhandle h, CBlasUplo uplo, size_t n,
   if (!hc::valid_uplo(uplo)) { *info = -2; return bad_arg(name, 2); }
   if (lda < n) { *info = -4; return bad_arg(name, 4); }
   if (n == 0) return CUDA_SUCCESS;
-  CUresult r = trtri_api<T>(name, h, uplo, CBlasNonUnit, n, A, lda, info);
-  if (r != CUDA_SUCCESS || *info != 0) return r;
-  return lauum_api<T>(name, h, uplo, n, A, lda, info);
+  hc::DeviceGuard g(h->device);
+  HC_CHECK(g.status());
+  return triangle_ops<T>(h, uplo, CBlasNonUnit, n, dptr<T>(A), lda, true, true, info);
 }
 
 template <typename T>
@@ -510,7 +581,7 @@ CUresult trti22_api(const char *name, CULAPACKhandle h, CBlasUplo uplo, CBlasDia
       HC_CHECK(hipMemsetAsync(dinfo, 0, sizeof(int), stream));
   }
   HC_CHECK(hc::diag_trtri<T>(stream, (char)uplo, (char)diag, (int)n, dptr<const T>(A), (long)lda,
-                             dptr<T>(B), (long)ldb, nullptr, 0, dinfo));
+                             dptr<T>(B), (long)ldb, dinfo));
   return CUDA_SUCCESS;
 }
 
