@@ -19,8 +19,8 @@ struct __cubatchedplan_st {
   char uplo;
   char precision;  // 'D' (FP64 storage) or 'S' (FP32 storage)
   int count;
-  int grid_inverse;        // persistent grid of the factor + inverse kernel
-  int reg_count[3], reg_grid[3];  // register-resident factor kernels: matrices and grid per size class
+  int reg_count[3], reg_grid[3];  // matrices per size class, grid of the factor kernels
+  int inv_grid[3];                // grid of the inverse kernels
   int *d_n;
   long *d_off;
   int *d_order;
@@ -35,22 +35,21 @@ struct __cubatchedplan_st {
 
 namespace {
 
+template <typename ST>
+hipError_t launch_as(const __cubatchedplan_st *p, hipStream_t s, CUdeviceptr A, double *logdet, int *info, bool inverse) {
+  ST *a = reinterpret_cast<ST *>(A);
+  HC_TRY(hc::potrf_batched_reg<ST>(s, p->uplo, p->d_cnt, p->reg_count, p->reg_grid, p->d_n, p->d_off, p->d_order, a,
+                                   logdet, info));
+  if (!inverse) return hipSuccess;
+  return hc::potri_batched_reg<ST>(s, p->uplo, p->d_cnt, p->reg_count, p->inv_grid, p->d_n, p->d_off, p->d_order, a,
+                                   info);
+}
+
 hipError_t launch(const __cubatchedplan_st *p, hipStream_t s, CUdeviceptr A, CUdeviceptr logdet,
                   CUdeviceptr info, bool inverse) {
   double *ld = reinterpret_cast<double *>(logdet);
   int *inf = reinterpret_cast<int *>(info);
-  if (!inverse) {
-    if (p->precision == 'D')
-      return hc::potrf_batched_reg<double>(s, p->uplo, p->d_cnt, p->reg_count, p->reg_grid, p->d_n, p->d_off,
-                                           p->d_order, reinterpret_cast<double *>(A), ld, inf);
-    return hc::potrf_batched_reg<float>(s, p->uplo, p->d_cnt, p->reg_count, p->reg_grid, p->d_n, p->d_off,
-                                        p->d_order, reinterpret_cast<float *>(A), ld, inf);
-  }
-  if (p->precision == 'D')
-    return hc::potrf_batched<double>(s, p->uplo, p->count, p->d_n, p->d_off, p->d_order,
-                                     reinterpret_cast<double *>(A), ld, inf, p->grid_inverse, true);
-  return hc::potrf_batched<float>(s, p->uplo, p->count, p->d_n, p->d_off, p->d_order,
-                                  reinterpret_cast<float *>(A), ld, inf, p->grid_inverse, true);
+  return p->precision == 'D' ? launch_as<double>(p, s, A, ld, inf, inverse) : launch_as<float>(p, s, A, ld, inf, inverse);
 }
 
 void release_graph(__cubatchedplan_st *p) {
@@ -148,25 +147,23 @@ CUresult cuPotrfBatchedPlanCreate(CULAPACKhandle h, CBlasUplo uplo, char precisi
   }
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return nv[a] > nv[b]; });
-  // persistent grid: at most every CU filled to the kernel's occupancy (a
-  // workgroup that waits for a slot would start its share late); fewer per CU
-  // when the autotuner measured that faster ($CUCHOLESKY_BATCHED_PER_CU
-  // overrides both)
+  // persistent grids: every CU filled to the kernel's occupancy (a workgroup
+  // that waits for a slot would start its share late); the inverse kernels
+  // take fewer per CU when the autotuner measured that faster
+  // ($CUCHOLESKY_BATCHED_PER_CU caps both)
   const char *env = std::getenv("CUCHOLESKY_BATCHED_PER_CU");
   const int forced = env != nullptr ? std::atoi(env) : 0;
-  auto per_cu = [&](bool inverse) {
-    const int occ = precision == 'D' ? hc::potrf_batched_blocks_per_cu<double>((char)uplo, inverse)
-                                     : hc::potrf_batched_blocks_per_cu<float>((char)uplo, inverse);
-    const int want = forced > 0 ? forced : hc::tuned_batched_per_cu(precision, inverse);
-    return want > 0 ? std::min(want, occ) : occ;
-  };
-  p->grid_inverse = std::max(1, std::min<int>((int)count, cus * per_cu(true)));
-  // register-resident factor kernels: every CU filled to their occupancy
+  const int tuned = hc::tuned_batched_per_cu(precision, true);
+  const int inv_cap = forced > 0 ? forced : (tuned > 0 ? tuned : 1 << 20);
   for (size_t i = 0; i < count; i++) p->reg_count[hc::batched_reg_class(nv[i])]++;
+  const bool dbl = precision == 'D';
   for (int c = 0; c < 3; c++) {
-    const int occ = precision == 'D' ? hc::potrf_batched_reg_blocks_per_cu<double>((char)uplo, c)
-                                     : hc::potrf_batched_reg_blocks_per_cu<float>((char)uplo, c);
+    const int occ = dbl ? hc::potrf_batched_reg_blocks_per_cu<double>((char)uplo, c)
+                        : hc::potrf_batched_reg_blocks_per_cu<float>((char)uplo, c);
+    const int inv = dbl ? hc::potri_batched_reg_blocks_per_cu<double>((char)uplo, c)
+                        : hc::potri_batched_reg_blocks_per_cu<float>((char)uplo, c);
     p->reg_grid[c] = cus * (forced > 0 ? std::min(forced, occ) : occ);
+    p->inv_grid[c] = cus * std::min(inv_cap, inv);
   }
   hipError_t e = hipMalloc(&p->d_cnt, 3 * sizeof(int));
   if (e == hipSuccess) e = hipMemcpy(p->d_cnt, p->reg_count, 3 * sizeof(int), hipMemcpyHostToDevice);

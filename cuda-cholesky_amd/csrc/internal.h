@@ -343,16 +343,6 @@ hipError_t trsm_multi(hipStream_t s, char uplo, char trans, long n, long nrhs, c
 // batched factorisation (batched.hip)
 // ---------------------------------------------------------------------------
 constexpr int kBatchedMaxN = 256;
-// resident workgroups per CU of the batched kernel (its occupancy)
-template <typename ST> int potrf_batched_blocks_per_cu(char uplo, bool inverse);
-// Factor count packed matrices in place (matrix order[t] for t = 0..count-1,
-// n = nvec[i] <= kBatchedMaxN, at element offset offs[i]); info[i] and
-// logdet[i] (may be null) per matrix; `grid` persistent workgroups.  With
-// `inverse`, each factored matrix is then overwritten by its inverse.
-template <typename ST>
-hipError_t potrf_batched(hipStream_t s, char uplo, int count, const int *nvec, const long *offs,
-                         const int *order, ST *A, double *logdet, int *info, int grid, bool inverse);
-
 // Register-resident factorisation + logdet (no inverse), in three size
 // classes (batched_reg_class: orders up to 64, up to 128, up to 256).
 // `order` lists class 2, then 1, then 0 (decreasing order); d_cnt[c] (device
@@ -364,6 +354,12 @@ template <typename ST>
 hipError_t potrf_batched_reg(hipStream_t s, char uplo, const int *d_cnt, const int *h_cnt, const int grid[3],
                              const int *nvec, const long *offs, const int *order, ST *A, double *logdet, int *info);
 template <typename ST> int potrf_batched_reg_blocks_per_cu(char uplo, int cls);
+// The factored matrices (info[i] == 0) overwritten by their inverses, with the
+// same size classes and arguments.
+template <typename ST>
+hipError_t potri_batched_reg(hipStream_t s, char uplo, const int *d_cnt, const int *h_cnt, const int grid[3],
+                             const int *nvec, const long *offs, const int *order, ST *A, const int *info);
+template <typename ST> int potri_batched_reg_blocks_per_cu(char uplo, int cls);
 // Resolves a device's copy of the no-allocation entry point's scratch array
 // (batched_noalloc.hip), once per device, with that device current.
 hipError_t noalloc_setup(int device);
