@@ -107,7 +107,7 @@ CUresult cuPotrfBatchedRun(CUbatchedplan plan, CUdeviceptr A, CUdeviceptr logdet
 /*
  * cuPotriBatchedRun: the same factorisation and logdet, then every factored
  * matrix (info[i] == 0) is overwritten by its inverse (triangle uplo of
- * A_i^-1, LAPACK xPOTRI semantics), in the same single launch.
+ * A_i^-1, LAPACK xPOTRI semantics), in the same graph launch.
  */
 CUresult cuPotriBatchedRun(CUbatchedplan plan, CUdeviceptr A, CUdeviceptr logdet, CUdeviceptr info,
                            CUstream stream);
