@@ -287,6 +287,7 @@ __device__ __forceinline__ double recip_chain(double d) {
 // count and its pivot chain: a column-at-a-time leaf in registers (rank-1
 // updates with one DPP broadcast and one FMA per column) takes 4306 cycles,
 // this one 2930 (one wave alone, real).
+// Only the real part of a diagonal entry is used (complex).
 // On return f holds L (entries above the diagonal unspecified).  The inverse
 // (zeros above the diagonal) is handed out block by block: sink(r, l, x) gets
 // l = L(lc, lg + 4 r) and x = X(lg + 4 r, lc) in lane lc + 16 lg.  Returns the
@@ -357,8 +358,11 @@ __device__ __forceinline__ int leaf_factor_invert(TileAcc<T> &f, Sink sink) {
     y[3] = submul(submul(submul(y[3], l30, y[0]), l31, y[1]), l32, y[2]);
     const T xr = rs * sel4(lg, y);        // row k of X
     if constexpr (r < 3) acc_rank4_sub(x, sel(lc > b + 3, lr, from_real<T>(0.0)), xr);
-    acc_set(L, r, lr);
-    sink(r, lr, xr);
+    // the diagonal is real: an imaginary part (the caller's, which is ignored, or
+    // rounding) stays in its own entry up to here
+    const T lf = is_complex<T>::value ? sel(lc == b + lg, from_real<T>(realx(lr)), lr) : lr;
+    acc_set(L, r, lf);
+    sink(r, lf, xr);
     __builtin_amdgcn_sched_barrier(0);
   });
   f = L;

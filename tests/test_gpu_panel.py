@@ -85,3 +85,35 @@ def test_potrf_failing_pivot(gpu, lapack, prec, uplo, value):
         W = store(A, uplo, n, dtype)
         st, info = getattr(gpu, f"cu{prec}potrf")(lapack, ord(uplo), n, gpu.ptr(W), n)
         assert st == 0 and info == k + 1, (k, info)
+
+
+def imaginary_diagonal(n, value):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    return 1.0 + 6.0 * torch.rand(n, generator=g, device="cuda", dtype=torch.float64) if value == "finite" \
+        else torch.full((n,), float("nan"), device="cuda", dtype=torch.float64)
+
+
+@pytest.mark.parametrize("prec", "CZ")
+@pytest.mark.parametrize("uplo", "LU")
+@pytest.mark.parametrize("n,value", [(n, "finite") for n in (1, 5, 16, 40, 64, 65, 150, 193)] +
+                         [(n, "nan") for n in (1, 5, 16, 40, 64)])
+def test_complex_diagonal_is_real(gpu, lapack, prec, uplo, n, value):
+    """The imaginary part of the input's diagonal is not used: the factor and
+    the inverse are those of the clean matrix to the bit, and their diagonals
+    are real exactly."""
+    dtype = TYPES[prec]
+    clean = store(spd(n, 3 * n + 2, dtype), uplo, n + 1, dtype)
+    dirty = clean.clone()
+    k = torch.arange(n, device="cuda")
+    torch.view_as_real(dirty)[k, k, 1] = imaginary_diagonal(n, value).to(torch.view_as_real(dirty).dtype)
+    got = []
+    for W in (clean, dirty):
+        st, info = getattr(gpu, f"cu{prec}potrf")(lapack, ord(uplo), n, gpu.ptr(W), n + 1)
+        assert st == 0 and info == 0
+        F = factor_of(W, n, uplo).clone()
+        st, info = getattr(gpu, f"cu{prec}potri")(lapack, ord(uplo), n, gpu.ptr(W), n + 1)
+        assert st == 0 and info == 0
+        X = factor_of(W, n, uplo).clone()
+        assert (F.diagonal().imag == 0).all() and (X.diagonal().imag == 0).all()
+        got.append((F, X))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
