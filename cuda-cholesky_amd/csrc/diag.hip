@@ -156,6 +156,7 @@ using t16::acc_zero;
 using t16::acc_load;
 using t16::acc_store;
 using t16::acc_get;
+using t16::acc_rank4_add;
 using t16::acc_rank4_sub;
 using t16::frag_load;
 using t16::frag_rank4;
@@ -823,69 +824,71 @@ panel_potrf_kernel(int m, int jb, ST *A, long lda, ST *ws, int *flags, int epoch
 // ---------------------------------------------------------------------------
 // Triangular inverse of one block in LDS (packed lower tiles as above, lower
 // form, unit diagonals stored as ones): the 16 x 16 diagonal tiles first, one
-// wave each, then pairs of inverted blocks of w = 1, 2, 4 tiles are joined,
-// X21 = -X22 L21 X11, every tile product on the matrix cores.  T = -X22 L21 is
-// formed in registers and written over L21 before the second product, so
-// nothing but the tiles is needed.  A column-by-column substitution in
-// registers (one barrier per column) took 108 us per launch, this one 17 us
-// (128 x 128 doubles).
+// wave each, then X = inv(L) by tile rows, S = sum_{J<=K<I} L_IK X_KJ and
+// L_II X_IJ = -S, one wave per tile column J (it reads row I of L, which nobody
+// needs after that, and its own column of X: one barrier per row).  The solve
+// with L_II is Y = -X_II S corrected once, Y -= X_II (S + L_II Y), from a copy
+// of L_II kept behind the tiles.
+// The inverse takes the place of L in solves, so its residual L X - I has to be
+// that of a substitution, whatever the grading of L.  Measured on the factor of
+// a squared-exponential covariance (n = 128, length 0.05, nugget 1e-8), residual
+// of the solve A x = b from both of its triangles: substitution element by
+// element 5e-14, this 4e-14, without the correction 1e-12, joining inverted
+// halves (X21 = -X22 L21 X11) 3e-13 (and 7e-11 in L X - I at nugget 1e-10).
+// Waves w and w + 4 share a SIMD and take columns w and 7 - w, so that every
+// matrix core has the same products.
 // ---------------------------------------------------------------------------
+template <int NMAX>
+constexpr int tri_lds_elems() {
+  constexpr int NP = NMAX / LEAF;
+  return (NP * (NP + 1) / 2 + NP) * LEAF * (LEAF + 1);
+}
+
 template <typename T, int NMAX>
 __device__ __forceinline__ void tiles_invert(T *S, int np) {
-  constexpr int NPMAX = NMAX / LEAF, LL = LEAF + 1, TS = LEAF * LL, NW = BLK_THREADS / 64;
-  constexpr int PER = (NPMAX * NPMAX / 4 + NW - 1) / NW;  // tiles per wave on the widest level
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int NPMAX = NMAX / LEAF, LL = LEAF + 1, TS = LEAF * LL;
+  static_assert(BLK_THREADS / 64 == 8 && NPMAX <= 8, "a wave per tile column");
+  const int lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   auto tile = [&](int I, int J) { return S + (I * (I + 1) / 2 + J) * TS; };
+  T *const Ld = S + NPMAX * (NPMAX + 1) / 2 * TS;  // L_II, zeros above the diagonal
   if (wave < np) {
-    T a[LEAF], x[4];
+    T a[LEAF], x[4], l[4];
     T *t = tile(wave, wave);
 #pragma unroll
-    for (int c = 0; c < LEAF; c++) a[c] = t[c * LL + (lane & 15)];
+    for (int c = 0; c < LEAF; c++) a[c] = t[c * LL + lc];
+#pragma unroll
+    for (int j = 0; j < 4; j++) l[j] = t16::sel(lg + 4 * j <= lc, t[(lg + 4 * j) * LL + lc], from_real<T>(0.0));
     t16::leaf_inverse_cols<T>(a, x);
 #pragma unroll
-    for (int j = 0; j < 4; j++) t[((lane >> 4) + 4 * j) * LL + (lane & 15)] = x[j];
+    for (int j = 0; j < 4; j++) {
+      t[(lg + 4 * j) * LL + lc] = x[j];
+      Ld[wave * TS + (lg + 4 * j) * LL + lc] = l[j];
+    }
   }
   __syncthreads();
-  for (int w = 1; w < np; w *= 2) {
-    // tile u of the level: pair u / w^2, row and column in the pair's block 21
-    const int lw = 31 - __builtin_clz(w);
-    auto place = [&](int u, int &i, int &j, int &mid) {
-      const int base = (u >> (2 * lw)) * 2 * w;
-      mid = base + w;
-      i = mid + ((u >> lw) & (w - 1));
-      j = base + (u & (w - 1));
-      return i < np;
-    };
-    TileAcc<T> acc[PER];
-#pragma unroll
-    for (int q = 0; q < PER; q++) {
-      int i, j, mid;
-      acc_zero(acc[q]);
-      if (place(wave + q * NW, i, j, mid))
-        for (int k = mid; k <= i; k++) tile_mma<false>(acc[q], tile(i, k), LL, tile(k, j), LL, -1.0);
-    }
+  const int J = wave < 4 ? wave : 11 - wave;
+  for (int I = 1; I < np; I++) {
+    TileAcc<T> s, y, xf, lf;
+    acc_zero(s);
+    if (J < I)
+      for (int K = J; K < I; K++) tile_mma<false>(s, tile(I, K), LL, tile(K, J), LL, 1.0);
     __syncthreads();
+    if (J < I) {
+      frag_load(xf, tile(I, I), LL);
+      frag_load(lf, Ld + I * TS, LL);
+      acc_zero(y);
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-      int i, j, mid;
-      if (place(wave + q * NW, i, j, mid)) acc_store(acc[q], tile(i, j), LL);
-    }
-    __syncthreads();
+      for (int q = 0; q < 4; q++) acc_rank4_sub(y, acc_get(xf, q), acc_get(s, q));
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-      int i, j, mid;
-      acc_zero(acc[q]);
-      if (place(wave + q * NW, i, j, mid))
-        for (int k = j; k < mid; k++) tile_mma<false>(acc[q], tile(i, k), LL, tile(k, j), LL, 1.0);
-    }
-    __syncthreads();
+      for (int q = 0; q < 4; q++) acc_rank4_add(s, acc_get(lf, q), acc_get(y, q));
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-      int i, j, mid;
-      if (place(wave + q * NW, i, j, mid)) acc_store(acc[q], tile(i, j), LL);
+      for (int q = 0; q < 4; q++) acc_rank4_sub(y, acc_get(xf, q), acc_get(s, q));
+      acc_store(y, tile(I, J), LL);
+      wave_lds_fence();
     }
-    __syncthreads();
   }
+  __syncthreads();
 }
 
 // Packed lower tiles of the n x n block at A: lower-form element (r, c) is
@@ -962,7 +965,7 @@ __global__ void __launch_bounds__(BLK_THREADS)
 diag_trtri_kernel(int lower, int unit, int ntot, int nb, const ST *A, long lda, ST *B, long ldb,
                   const int *abort_flag) {
   if (abort_flag != nullptr && *abort_flag != 0) return;
-  __shared__ T S[diag_lds_elems<NMAX>()];
+  __shared__ T S[tri_lds_elems<NMAX>()];
   const long off = (long)blockIdx.x * nb;
   const int n = (int)min((long)nb, (long)ntot - off);
   A += off * lda + off;
@@ -1020,7 +1023,7 @@ __global__ void __launch_bounds__(256) tri_copy_kernel(int lower, int n, const T
 template <typename T, typename ST, int NMAX>
 __global__ void __launch_bounds__(BLK_THREADS)
 trsm_inv_kernel(int lowerlike, int op, int unit, long m, int nb, const ST *A, long lda, ST *W) {
-  __shared__ T S[diag_lds_elems<NMAX>()];
+  __shared__ T S[tri_lds_elems<NMAX>()];
   const long off = (long)blockIdx.x * nb;
   const int n = (int)((m - off) < nb ? (m - off) : nb);
   // lower form: op(A)(r, c) when op(A) is lower-like, else conj(op(A)(c, r));

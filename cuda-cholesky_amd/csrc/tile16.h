@@ -188,8 +188,8 @@ __device__ __forceinline__ void frag_store(const TileAcc<T> &f, T *C, int ls) {
 }
 
 // Rank-4 pieces (k-step s of the operands).  frag: f (row fragments) += or
-// -= A conj(B)^T with A, B row fragments; acc: c (result layout) -= L X with
-// L row fragments and X in the result layout.
+// -= A conj(B)^T with A, B row fragments; acc: c (result layout) -= or += L X
+// with L row fragments and X in the result layout.
 template <bool NEG>
 __device__ __forceinline__ void frag_rank4(TileAcc<double> &f, double a, double b) {
   f.re = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, f.re, 0, 0, NEG ? kNegA : 0);
@@ -209,6 +209,16 @@ __device__ __forceinline__ void acc_rank4_sub(TileAcc<zd> &c, zd a, zd x) {
   c.im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, x.y, c.im, 0, 0, kNegA);
   c.re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, x.y, c.re, 0, 0, 0);
   c.im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, x.x, c.im, 0, 0, kNegA);
+}
+
+__device__ __forceinline__ void acc_rank4_add(TileAcc<double> &c, double a, double x) {
+  c.re = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x, c.re, 0, 0, 0);
+}
+__device__ __forceinline__ void acc_rank4_add(TileAcc<zd> &c, zd a, zd x) {
+  c.re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, x.x, c.re, 0, 0, 0);
+  c.im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, x.y, c.im, 0, 0, 0);
+  c.re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, x.y, c.re, 0, 0, kNegA);
+  c.im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, x.x, c.im, 0, 0, 0);
 }
 
 // o[j] = v of lane l % 16 + 16 j: every lane gets the four values that its

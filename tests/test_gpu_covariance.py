@@ -1,0 +1,107 @@
+"""Residuals on graded factors: squared-exponential covariances.
+
+The Cholesky factor of exp(-(x - y)^2 / (2 l^2)) + nugget I on a grid has
+columns that fall by orders of magnitude, so that a product with the inverse of
+a block loses digits where a substitution does not; matrices of independent
+entries do not show it.  The bars are 10 n eps times the norms of the factors of
+the residual, with no condition number: a row-by-row substitution meets them
+with two digits to spare.
+"""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_panel import TYPES, factor_of, store
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(np.float64).eps
+
+
+def covariance(n, length, nugget, dtype):
+    x = torch.linspace(0.0, 1.0, n, device="cuda", dtype=torch.float64)
+    A = torch.exp(-((x[:, None] - x) ** 2) / (2.0 * length * length)) + nugget * torch.eye(n, device="cuda", dtype=torch.float64)
+    if not dtype.is_complex:
+        return A
+    k = torch.arange(n, device="cuda", dtype=torch.float64)
+    p = torch.polar(torch.ones_like(k), 0.37 * k * k)        # D A D^H: the same grading, complex entries
+    A = p[:, None] * A * p.conj()
+    A = torch.tril(A) + torch.tril(A, -1).mH
+    A.diagonal().imag.zero_()
+    return A
+
+
+def norm(M):
+    return torch.linalg.norm(M).item()
+
+
+def lower_factor(n, length, nugget, dtype):
+    return torch.linalg.cholesky(covariance(n, length, nugget, dtype))
+
+
+@pytest.mark.parametrize("prec", "DZ")
+@pytest.mark.parametrize("uplo", "LU")
+@pytest.mark.parametrize("n", [20, 60, 64, 100, 128])
+def test_trsm_residual(gpu, blas, prec, uplo, n):
+    """L X = B, from L and from U = L^H: the sides that a substitution solves
+    with a residual free of the condition number."""
+    dtype = TYPES[prec]
+    L = lower_factor(n, 0.05, 1e-10, dtype)
+    W = store(L if uplo == "L" else L.mH, uplo, n + 1, dtype)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    B = torch.randn(20, n, 2, generator=g, device="cuda", dtype=torch.float64)
+    B = torch.view_as_complex(B) if dtype.is_complex else B[..., 0].contiguous()
+    X = B.clone()
+    trans = gpu.NoTrans if uplo == "L" else (gpu.ConjTrans if dtype.is_complex else gpu.Trans)
+    st = getattr(gpu, f"cu{prec}trsm")(blas, gpu.Left, ord(uplo), trans, gpu.NonUnit, n, 20, 1.0, gpu.ptr(W), n + 1,
+                                       gpu.ptr(X), n, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert st == 0
+    err = norm(L @ X.mT - B.mT) / (norm(L) * norm(X) + norm(B))
+    assert err <= 10 * n * EPS, err
+
+
+@pytest.mark.parametrize("uplo", "LU")
+@pytest.mark.parametrize("prec,n", [(p, n) for p in "DZ" for n in (20, 48, 60, 64, 100, 128) if p == "D" or n <= 64])
+def test_trtri_residual(gpu, lapack, prec, uplo, n):
+    """||L X - I|| of one diagonal block (up to 64 complex, 128 real)."""
+    L = lower_factor(n, 0.05, 1e-10, TYPES[prec])
+    W = store(L if uplo == "L" else L.mH, uplo, n + 1, TYPES[prec])
+    st, info = getattr(gpu, f"cu{prec}trtri")(lapack, ord(uplo), gpu.NonUnit, n, gpu.ptr(W), n + 1)
+    torch.cuda.synchronize()
+    assert st == 0 and info == 0
+    X = factor_of(W, n, uplo)
+    err = norm(L @ X - torch.eye(n, device="cuda", dtype=X.dtype)) / (norm(L) * norm(X))
+    assert err <= 10 * n * EPS, err
+
+
+@pytest.mark.parametrize("uplo", "LU")
+@pytest.mark.parametrize("n,length,nugget", [(60, 0.05, 1e-8), (128, 0.05, 1e-8), (512, 0.05, 1e-10)])
+def test_potrs_residual(gpu, lapack, uplo, n, length, nugget):
+    A = covariance(n, length, nugget, torch.float64)
+    W = store(A, uplo, n + 1, torch.float64)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    B = torch.randn(20, n, generator=g, device="cuda", dtype=torch.float64)
+    X = B.clone()
+    st, info = gpu.cuDpotrf(lapack, ord(uplo), n, gpu.ptr(W), n + 1)
+    assert st == 0 and info == 0
+    st, info = gpu.cuDpotrs(lapack, ord(uplo), n, 20, gpu.ptr(W), n + 1, gpu.ptr(X), n)
+    torch.cuda.synchronize()
+    assert st == 0 and info == 0
+    err = norm(A @ X.mT - B.mT) / (norm(A) * norm(X) + norm(B))
+    assert err <= 10 * n * EPS, err
+
+
+@pytest.mark.parametrize("uplo", "LU")
+@pytest.mark.parametrize("n", [60, 100, 128])
+def test_potri_residual(gpu, lapack, uplo, n):
+    A = covariance(n, 0.1, 1e-8, torch.float64)
+    W = store(A, uplo, n + 1, torch.float64)
+    st, info = gpu.cuDpotrf(lapack, ord(uplo), n, gpu.ptr(W), n + 1)
+    assert st == 0 and info == 0
+    st, info = gpu.cuDpotri(lapack, ord(uplo), n, gpu.ptr(W), n + 1)
+    torch.cuda.synchronize()
+    assert st == 0 and info == 0
+    X = factor_of(W, n, uplo)
+    X = torch.tril(X) + torch.tril(X, -1).mH
+    err = norm(A @ X - torch.eye(n, device="cuda", dtype=X.dtype)) / (norm(A) * norm(X))
+    assert err <= 10 * n * EPS, err
