@@ -533,6 +533,9 @@ __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
         if constexpr (CPLX) v = cmake<T>(acc[0][i][j][r], acc[1][i][j][r]);
         else v = acc[0][i][j][r];
         v = p.alpha * v;
+        if constexpr (CPLX) {  // the imaginary part of a Hermitian diagonal is not used
+          if (p.real_diag && gm == gn) cv[j][r].y = 0.0;
+        }
         if (need_c && i * BJ + j >= npre) v = v + p.beta * cv[j][r];
         if constexpr (CPLX) {
           if (p.real_diag && gm == gn) v.y = 0.0;

@@ -114,7 +114,7 @@ inline int op_code(char t) { return t == 'N' ? OP_N : (t == 'T' ? OP_T : OP_C); 
 struct GemmOpts {
   int tri_out = TRI_NONE;   // write only row >= col (lower) or row <= col (upper)
   bool tri_grid = false;    // launch only tiles meeting the tri_out triangle (m == n)
-  bool real_diag = false;   // HERK: force the diagonal of D to be real
+  bool real_diag = false;   // HERK: C's diagonal is taken as real, D's is
   int tri_a = TRI_NONE;     // op(A) is triangular (lower- or upper-like): TRMM left
   int tri_b = TRI_NONE;     // op(B) is triangular: TRMM right
   bool unit = false;        // the triangular operand has an implicit unit diagonal

@@ -111,6 +111,7 @@ hipError_t factor_panel(CULAPACKhandle h, hipStream_t s, bool lower, long n, T *
     if (rem > 0 && !left) {
       hc::GemmOpts u;
       u.abort_flag = h->dinfo;
+      u.real_diag = hc::is_complex<T>::value;
       if (lower) {
         u.tri_out = hc::TRI_LOWER;
         HC_TRY(hc::gemm<T>(s, hc::OP_N, conj_op<T>(), rest, rem, ib, mone, at(r0, jj), lda,
@@ -271,6 +272,7 @@ hipError_t potrf_device(CULAPACKhandle h, char uplo, long n, T *A, long lda, T *
     hc::GemmOpts u;
     u.abort_flag = h->dinfo;
     u.bf16 = bf16;
+    u.real_diag = hc::is_complex<T>::value;
     // The next panel's update needs this panel and the previous trailing
     // update; the trailing update beyond the next panel needs only those
     // too.  On the look-ahead stream (ahead of the next panel's

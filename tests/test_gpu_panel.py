@@ -96,7 +96,7 @@ def imaginary_diagonal(n, value):
 @pytest.mark.parametrize("prec", "CZ")
 @pytest.mark.parametrize("uplo", "LU")
 @pytest.mark.parametrize("n,value", [(n, "finite") for n in (1, 5, 16, 40, 64, 65, 150, 193)] +
-                         [(n, "nan") for n in (1, 5, 16, 40, 64)])
+                         [(n, "nan") for n in (1, 5, 16, 40, 64, 65, 150, 193, 700, 1100)])
 def test_complex_diagonal_is_real(gpu, lapack, prec, uplo, n, value):
     """The imaginary part of the input's diagonal is not used: the factor and
     the inverse are those of the clean matrix to the bit, and their diagonals
@@ -117,3 +117,23 @@ def test_complex_diagonal_is_real(gpu, lapack, prec, uplo, n, value):
         assert (F.diagonal().imag == 0).all() and (X.diagonal().imag == 0).all()
         got.append((F, X))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("prec", "CZ")
+@pytest.mark.parametrize("uplo", "LU")
+@pytest.mark.parametrize("n,k", [(5, 3), (64, 40), (150, 64)])
+def test_herk_ignores_imaginary_diagonal(gpu, blas, prec, uplo, n, k):
+    """C's diagonal is real by definition: NaN in its imaginary part changes nothing."""
+    dtype = TYPES[prec]
+    A = torch.randn(k, n, device="cuda", dtype=dtype)
+    clean = store(spd(n, n, dtype), uplo, n, dtype)
+    dirty = clean.clone()
+    i = torch.arange(n, device="cuda")
+    torch.view_as_real(dirty)[i, i, 1] = float("nan")
+    for W in (clean, dirty):
+        st = getattr(gpu, f"cu{prec}herk")(blas, ord(uplo), gpu.NoTrans, n, k, -0.5, gpu.ptr(A), n, 0.75, gpu.ptr(W), n,
+                                           torch.cuda.current_stream().cuda_stream)
+        assert st == 0
+    torch.cuda.synchronize()
+    assert torch.equal(factor_of(clean, n, uplo), factor_of(dirty, n, uplo))
+    assert (factor_of(dirty, n, uplo).diagonal().imag == 0).all()
