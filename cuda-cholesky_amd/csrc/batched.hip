@@ -387,25 +387,33 @@ potrf_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
 // Register-resident inverse of factored matrices (info = 0): A^-1 = X^T X,
 // X = inv(L), in place over the factor.
 //
-// np = ceil(n / 16) tile columns; wave w of NPMAX / 2 owns columns w and
-// np - 1 - w of X (np + 1 tiles together, equal work), held in registers in the
-// matrix-core result layout, which is also the operand layout of the second
-// factor of every product here, so a column never moves between lanes.
+// np = ceil(n / 16) tile rows and columns; wave w of NPMAX / 2 owns first rows
+// np - 1 - w and w of X, then columns w and np - 1 - w of the result (np + 1
+// tiles together, equal work), held in registers in the matrix-core result
+// layout (rows: transposed), which is also the operand layout of the second
+// factor of every product here, so a tile never moves between lanes.
 //   * the waves invert the diagonal leaves into LDS;
-//   * each wave substitutes its columns, X_IJ = -X_II sum_{J<=K<I} L_IK X_KJ,
-//     with the tiles of L read from the matrix as operand fragments: no
-//     exchange between waves;
-//   * the columns replace L in the matrix, and each wave forms its columns of
-//     the result, R_ij = sum_{K>=i} X_Ki^T X_Kj, i ascending, with X_Ki from the
-//     matrix; R_ij takes the registers of X_ij, which no later i needs;
+//   * each wave forms its rows right to left, X_IJ = -(sum_{J<K<=I} X_IK L_KJ)
+//     X_JJ, with the tiles of L read from the matrix as operand fragments: no
+//     exchange between waves.  k runs as 4 lk + s there, so that in lower
+//     storage a lane's four elements are one load, and so are its four of X;
+//   * the rows replace L in the matrix, the waves read their columns of X back,
+//     and form their columns of the result, R_ij = sum_{K>=i} X_Ki^T X_Kj,
+//     i ascending, with X_Ki from the matrix; R_ij takes the registers of X_ij,
+//     which no later i needs;
 //   * R replaces X in the matrix.
-// Factor and inverse of 20000 matrices, n in [8, 256], FP32 storage: 9.8 ms with
-// a 4-wave workgroup that streams every tile of a matrix through memory at
-// every step, 7.4 ms with the register-resident factor (2.4 ms) and this kernel
-// (n > 128: 4.6 ms).  There the matrix cores are busy 20 % of the time
-// (SQ_VALU_MFMA_BUSY_CYCLES); the fully unrolled tile products are more code
-// than the instruction cache holds, but rolled loops over K spilled 200 to 800
-// registers (the columns are indexed at compile time).
+// X by rows has a small X L - I, which is what A X^T X - I needs.  By columns
+// (X_IJ = -X_II sum L_IK X_KJ, small L X - I) the columns would stay where they
+// are, but the residual of the inverse on graded factors is 30 to 500 times
+// larger: squared-exponential covariances, nugget 1e-8, ||A R - I|| / (||A||
+// ||R||) 3e-15 by rows, 2e-12 by columns at n = 128.
+// Factor and inverse of 20000 matrices, n in [8, 256]: FP32 storage 6.6 ms
+// (upper 6.7), of which the factor 2.4 (2.6), FP64 8.0 ms (8.3); by columns 7.5
+// (7.0) and 7.8 ms (9.2); a 4-wave workgroup that streams every tile of a matrix
+// through memory at every step 9.8 (8.4) and 11.1 ms (10.8).  The fully
+// unrolled tile products are more code than the instruction cache holds, but
+// rolled loops over K spilled 200 to 800 registers (rows and columns are indexed
+// at compile time).
 // ---------------------------------------------------------------------------
 template <typename ST, bool LOWER, int CLS, int NPMAX = RegClass<CLS>::NPMAX>
 __global__ void __launch_bounds__(NPMAX / 2 * 64) __attribute__((amdgpu_waves_per_eu(CLS == 0 ? 3 : 2, 8)))
@@ -431,18 +439,118 @@ potri_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
       for (int j = 0; j < 4; j++) D[I * LEAF * LL + (lk + 4 * j) * LL + li] = x[j];
     }
     __syncthreads();
-    // lane offsets of an operand fragment of a tile: element (row li, column
-    // lk + 4 s) for L, (row lk + 4 s, column li) for X^T; rows of the last tile
-    // row beyond n are read from a valid address and replaced by zero
-    const int rl = min(li, n - 1 - (np - 1) * LEAF);  // row within the last tile row, clamped
-    const unsigned ol = LOWER ? lk * n + li : li * n + lk, oe = LOWER ? lk * n + rl : rl * n + lk;
-    const unsigned ox = LOWER ? li * n + lk : lk * n + li;
-    v4d Z[NPMAX + 1];  // column w: tile w + t at t; column np - 1 - w: its tile t at NPMAX - t
-    // fn(sec, J, dmax) for the wave's columns
-    auto columns = [&](auto fn) __attribute__((always_inline)) {
-      if (2 * wave < np) fn(std::integral_constant<int, 0>{}, wave);
-      if (2 * wave + 1 < np) fn(std::integral_constant<int, 1>{}, np - 1 - wave);
+    // lane offsets in a tile: elements (row li, column lk) and (row lk, column li)
+    const unsigned ol = LOWER ? lk * n + li : li * n + lk, ox = LOWER ? li * n + lk : lk * n + li;
+    const int rstep = LOWER ? 4 : 4 * n, cstep = LOWER ? 4 * n : 4;  // four rows, four columns on
+    auto tile_at = [&](int I, int J) { return v.M + (LOWER ? (long)J * LEAF * n + I * LEAF : (long)I * LEAF * n + J * LEAF); };
+    // elements (row lk + 4 s, column li) of tile (K, J), the operand fragment of
+    // its transpose: a whole tile, or one with rows beyond n, which are zero
+    auto load_t = [&](int K, int J, auto &l) __attribute__((always_inline)) {
+      const ST *p = tile_at(K, J);
+#pragma unroll
+      for (int s = 0; s < 4; s++) l[s] = (double)p[s * rstep + ox];
     };
+    auto load_edge = [&](int K, int J, auto &l) __attribute__((always_inline)) {
+      const ST *p = tile_at(K, J);
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const bool ok = K * LEAF + lk + 4 * s < n;
+        const double x = (double)p[ok ? s * rstep + ox : 0u];
+        l[s] = ok ? x : 0.0;
+      }
+    };
+    // a tile of X that is whole (all but a ragged last tile row) and that lies
+    // along columns in memory is kept transposed there, so that the loads of
+    // X_Ki^T below run along memory; X_JJ stays in LDS
+    auto transposed = [&](int I) { return LOWER && (I + 1) * LEAF <= n; };
+    auto load_x = [&](int K, int J, auto &l) __attribute__((always_inline)) {
+      if (transposed(K)) {
+        const ST *p = tile_at(K, J);
+#pragma unroll
+        for (int s = 0; s < 4; s++) l[s] = (double)p[s * cstep + ol];
+      } else if (!LOWER && (K + 1) * LEAF <= n) {
+        load_t(K, J, l);
+      } else {
+        load_edge(K, J, l);
+      }
+    };
+    // rows 4 lk .. 4 lk + 3 of column li of tile (K, J) of L, contiguous in lower
+    // storage: the operand fragment of its transpose for products whose k runs
+    // as 4 lk + s; rows beyond n are zero
+    typedef ST row4 __attribute__((ext_vector_type(4), aligned(sizeof(ST))));
+    const unsigned of = LOWER ? li * n + 4 * lk : 4 * lk * n + li;
+    const int fstep = LOWER ? 1 : n;
+    auto load_l = [&](int K, int J, auto &l) __attribute__((always_inline)) {
+      const ST *p = tile_at(K, J) + of;
+      if (LOWER) {
+        const row4 x = *reinterpret_cast<const row4 *>(p);
+#pragma unroll
+        for (int s = 0; s < 4; s++) l[s] = (double)x[s];
+      } else {
+#pragma unroll
+        for (int s = 0; s < 4; s++) l[s] = (double)p[s * fstep];
+      }
+    };
+    auto load_l_edge = [&](int K, int J, auto &l) __attribute__((always_inline)) {
+      const ST *p = tile_at(K, J);
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const bool ok = K * LEAF + 4 * lk + s < n;
+        const double x = (double)p[ok ? of + s * fstep : 0u];
+        l[s] = ok ? x : 0.0;
+      }
+    };
+    v4d Z[NPMAX + 1];  // the long row or column: its tile t from the diagonal at t; the short one: at NPMAX - t
+    const int lp = 4 * (li & 3) + (li >> 2);  // rows of a result in the order 4 lk + r: from operand rows in this order
+    auto sections = [&](int longer, int shorter, auto fn) __attribute__((always_inline)) {
+      if (2 * wave < np) fn(std::integral_constant<int, 0>{}, longer);
+      if (2 * wave + 1 < np) fn(std::integral_constant<int, 1>{}, shorter);
+    };
+    auto rows = [&](auto fn) __attribute__((always_inline)) { sections(np - 1 - wave, wave, fn); };
+    auto columns = [&](auto fn) __attribute__((always_inline)) { sections(wave, np - 1 - wave, fn); };
+    rows([&](auto Sec, int I) __attribute__((always_inline)) {
+      constexpr int sec = decltype(Sec)::value, TM = sec ? NPMAX / 2 : NPMAX;
+      auto at = [](int u) { return sec ? NPMAX - u : u; };
+#pragma unroll
+      for (int r = 0; r < 4; r++) Z[at(0)][r] = D[I * LEAF * LL + (4 * lk + r) * LL + li];
+      t16::static_for<1, TM>([&](auto Dc) {
+        constexpr int d = decltype(Dc)::value;
+        if (d > I) return;
+        const int J = I - d;
+        v4d S = {0.0, 0.0, 0.0, 0.0}, acc = {0.0, 0.0, 0.0, 0.0};
+        t16::static_for<0, d>([&](auto Uc) {  // K = I - u
+          constexpr int u = decltype(Uc)::value;
+          double l[4];
+          if (u == 0 && I == np - 1) load_l_edge(I, J, l);
+          else load_l(I - u, J, l);
+#pragma unroll
+          for (int s = 0; s < 4; s++) S = __builtin_amdgcn_mfma_f64_16x16x4f64(l[s], Z[at(u)][s], S, 0, 0, 0);
+        });
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(D[J * LEAF * LL + lp * LL + lk + 4 * s], S[s], acc, 0, 0, kNegA);
+        Z[at(d)] = acc;
+      });
+    });
+    __syncthreads();  // every read of L is done
+    rows([&](auto Sec, int I) __attribute__((always_inline)) {
+      constexpr int sec = decltype(Sec)::value, TM = sec ? NPMAX / 2 : NPMAX;
+      t16::static_for<1, TM>([&](auto Dc) {
+        constexpr int d = decltype(Dc)::value;
+        if (d > I) return;
+        const int J = I - d;
+        const v4d &z = Z[sec ? NPMAX - d : d];
+        // X(li, 4 lk + r): along memory in upper storage, and in lower storage where the tile is transposed
+        if ((I + 1) * LEAF <= n) {
+          const row4 x = {(ST)z[0], (ST)z[1], (ST)z[2], (ST)z[3]};
+          *reinterpret_cast<row4 *>(tile_at(I, J) + li * n + 4 * lk) = x;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; r++) v.put(I * LEAF + li, J * LEAF + 4 * lk + r, z[r]);
+        }
+      });
+    });
+    __syncthreads();
     columns([&](auto Sec, int J) __attribute__((always_inline)) {
       constexpr int sec = decltype(Sec)::value, TM = sec ? NPMAX / 2 : NPMAX;
       auto at = [](int u) { return sec ? NPMAX - u : u; };
@@ -450,50 +558,9 @@ potri_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
       for (int r = 0; r < 4; r++) Z[at(0)][r] = D[J * LEAF * LL + li * LL + lk + 4 * r];
       t16::static_for<1, TM>([&](auto Dc) {
         constexpr int d = decltype(Dc)::value;
-        if (J + d >= np) return;
-        const int I = J + d;
-        const bool edge = I == np - 1, ok = I * LEAF + li < n;
-        const unsigned o = edge ? oe : ol;
-        v4d S = {0.0, 0.0, 0.0, 0.0}, acc = {0.0, 0.0, 0.0, 0.0};
-        t16::static_for<0, d>([&](auto Uc) {
-          constexpr int u = decltype(Uc)::value;
-          const int K = J + u;
-          const ST *p = v.M + (LOWER ? (long)K * LEAF * n + I * LEAF : (long)I * LEAF * n + K * LEAF);
-          double l[4];
-#pragma unroll
-          for (int s = 0; s < 4; s++) l[s] = (double)p[(LOWER ? 4 * s * n : 4 * s) + o];
-#pragma unroll
-          for (int s = 0; s < 4; s++)
-            S = __builtin_amdgcn_mfma_f64_16x16x4f64(ok ? l[s] : 0.0, Z[at(u)][s], S, 0, 0, 0);
-        });
-#pragma unroll
-        for (int s = 0; s < 4; s++)
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(D[I * LEAF * LL + (lk + 4 * s) * LL + li], S[s], acc, 0, 0, kNegA);
-        Z[at(d)] = acc;
+        if (J + d < np) load_x(J + d, J, Z[at(d)]);
       });
     });
-    // a tile of X that is whole (all but a ragged last tile row) and that lies
-    // along columns in memory is kept transposed there, so that both its
-    // stores and the loads of X_Ki^T below run along memory; X_JJ stays in LDS
-    auto transposed = [&](int I) { return LOWER && (I + 1) * LEAF <= n; };
-    __syncthreads();  // every read of L is done
-    columns([&](auto Sec, int J) __attribute__((always_inline)) {
-      constexpr int sec = decltype(Sec)::value, TM = sec ? NPMAX / 2 : NPMAX;
-      t16::static_for<1, TM>([&](auto Dc) {
-        constexpr int d = decltype(Dc)::value;
-        if (J + d >= np) return;
-        const int I = J + d;
-        if (transposed(I)) {
-          ST *p = v.M + (long)J * LEAF * n + I * LEAF;
-#pragma unroll
-          for (int r = 0; r < 4; r++) p[4 * r * n + ol] = (ST)Z[sec ? NPMAX - d : d][r];
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; r++) v.put(I * LEAF + lk + 4 * r, J * LEAF + li, Z[sec ? NPMAX - d : d][r]);
-        }
-      });
-    });
-    __syncthreads();
     columns([&](auto Sec, int J) __attribute__((always_inline)) {
       constexpr int sec = decltype(Sec)::value, TM = sec ? NPMAX / 2 : NPMAX;
       auto at = [](int u) { return sec ? NPMAX - u : u; };
@@ -508,21 +575,8 @@ potri_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
         t16::static_for<d + 1, TM>([&](auto Uc) {
           constexpr int u = decltype(Uc)::value;
           if (J + u >= np) return;
-          const int K = J + u;
-          const ST *p = v.M + (LOWER ? (long)i * LEAF * n + K * LEAF : (long)K * LEAF * n + i * LEAF);
           double l[4];
-          if (transposed(K)) {
-#pragma unroll
-            for (int s = 0; s < 4; s++) l[s] = (double)p[4 * s * n + ol];
-          } else {
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-              const bool ok = K * LEAF + lk + 4 * s < n;
-              const unsigned o = ox + (LOWER ? 4 * s : 4 * s * n);
-              const double x = (double)p[ok ? o : 0u];
-              l[s] = ok ? x : 0.0;
-            }
-          }
+          load_x(J + u, i, l);
 #pragma unroll
           for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(l[s], Z[at(u)][s], acc, 0, 0, 0);
         });

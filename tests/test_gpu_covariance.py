@@ -105,3 +105,26 @@ def test_potri_residual(gpu, lapack, uplo, n):
     X = torch.tril(X) + torch.tril(X, -1).mH
     err = norm(A @ X - torch.eye(n, device="cuda", dtype=X.dtype)) / (norm(A) * norm(X))
     assert err <= 10 * n * EPS, err
+
+
+@pytest.mark.parametrize("uplo", "LU")
+def test_batched_inverse_residual(gpu, lapack, uplo):
+    """The three size classes of the batched plan, at their edges."""
+    cases = [(16, 0.1), (17, 0.1), (60, 0.1), (64, 0.1), (65, 0.1), (100, 0.1), (128, 0.1), (129, 0.05), (250, 0.02),
+             (256, 0.02)]
+    mats = [covariance(n, length, 1e-8, torch.float64) for n, length in cases]
+    sizes = [n for n, _ in cases]
+    offs = [int(v) for v in np.cumsum([0] + [n * n for n in sizes[:-1]])]
+    W = torch.cat([M.reshape(-1) for M in mats])
+    logdet = torch.zeros(len(sizes), device="cuda", dtype=torch.float64)
+    info = torch.full((len(sizes),), -9, device="cuda", dtype=torch.int32)
+    with gpu.BatchedPlan(lapack, ord(uplo), "D", sizes, offs) as plan:
+        assert plan.status == 0
+        assert plan.run_inverse(gpu.ptr(W), gpu.ptr(logdet), gpu.ptr(info), torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+    assert (info == 0).all()
+    for n, o, A in zip(sizes, offs, mats):
+        X = factor_of(W[o:o + n * n].reshape(n, n), n, uplo)
+        X = torch.tril(X) + torch.tril(X, -1).mT
+        err = norm(A @ X - torch.eye(n, device="cuda", dtype=X.dtype)) / (norm(A) * norm(X))
+        assert err <= 10 * n * EPS, (n, err)
