@@ -203,10 +203,6 @@ __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
   using PA = LoadPattern<MT, TA == OP_N>;
   using PB = LoadPattern<NT, TB != OP_N>;
   constexpr int EA = PA::E, EB = PB::E;
-  // Register sets of the operand loads in flight.  Two for the 64 x 64 complex
-  // tile or three for the 64 x 64 real one measured no faster (n = 1024
-  // inverse 714 us either way, zpotrf + zpotri n = 8192 44.6 ms).
-  constexpr int NSET = 1;
   static_assert(EA >= 1 && EB >= 1 && BI >= 1 && BJ >= 1, "tile too small");
 
   __shared__ R sA[2 * BUFA];
@@ -352,7 +348,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
     constexpr int SA_Q = PA::KSTEP * LSA + PA::RSTEP;
     constexpr int SB_Q = PB::KSTEP * LSB + PB::RSTEP;
 
-    T ra[NSET][EA], rb[NSET][EB];
+    T ra[EA], rb[EB];
     // Out-of-range elements read a valid address (the operand's origin) and
     // are replaced by zero, so the loads carry no branches.
     // Interior tiles take unpredicated loads on every whole K step that does
@@ -360,12 +356,12 @@ __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
     // cut to the triangle, so such a step lies strictly inside it.  Edge
     // tiles, diagonal steps and a partial last step check every element.
     // (With the last step's raggedness taken for the whole range, every step
-    // of a product with k % 16 != 0 was checked: DGEMM 5003 x 1501 x 2999
-    // 45 TFLOP/s, now 50.)
-    const bool interior = m0 + MT <= p.m && n0 + NT <= p.n;
+    // of a product with k % 16 != 0 is checked: DGEMM 5003 x 1501 x 2999
+    // 46 TFLOP/s, so 51.)
+    const bool interior = m0 + MT <= p.m && n0 + NT <= p.n, whole = (kend - kbeg) % KT == 0;
     const bool tri_ops = p.tri_a != TRI_NONE || p.tri_b != TRI_NONE;
-    auto load = [&](int kt_off, const T *qa, const T *qb, T (&ra)[EA], T (&rb)[EB]) __attribute__((always_inline)) {
-      bool fast = interior && kbeg + kt_off + KT <= kend;
+    auto load = [&](int kt_off, const T *qa, const T *qb) __attribute__((always_inline)) {
+      bool fast = interior && (whole || kbeg + kt_off + KT <= kend);
       if (tri_ops) {
         const int k0 = kbeg + kt_off;
         fast = fast && (p.tri_a == TRI_NONE || k0 + KT <= m0 || k0 >= m0 + MT) &&
@@ -407,7 +403,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
         rb[q] = v;
       }
     };
-    auto store = [&](int buf, const T (&ra)[EA], const T (&rb)[EB]) __attribute__((always_inline)) {
+    auto store = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
       for (int q = 0; q < EA; q++) lds_put(sA + buf * BUFA, PSA, sa0 + q * SA_Q, ra[q]);
 #pragma unroll
@@ -415,28 +411,28 @@ __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
     };
 
     const int ntiles = (kend - kbeg + KT - 1) / KT;
-    // Step kt + NSET is requested into the register set of step kt while step
-    // kt is multiplied from LDS, so NSET steps are in flight.
-    load(0, pa, pb, ra[0], rb[0]);
+    load(0, pa, pb);
     seed_c();
-#pragma unroll
-    for (int u = 1; u < NSET; u++)
-      if (u < ntiles) {
-        pa += a_kstride;
-        pb += b_kstride;
-        load(u * KT, pa, pb, ra[u], rb[u]);
-      }
-    store(0, ra[0], rb[0]);
+    store(0);
     __syncthreads();
-    for (int kb = 0; kb < ntiles; kb += NSET)
+    // One K step per outer trip.  The inner loop of one trip is for the compiler,
+    // which otherwise schedules a ragged range as if every step were checked
+    // (DGEMM 300 x 300 x 3000, T N: 200 us, as one plain loop 300 us; 5003 x 1501 x
+    // 2999, N T: 880 and 970 us).  `whole` keeps the test of the last step out
+    // of the ranges that do not need it (4096 x 4096 x 1024, T N: 532 us, tested
+    // 557 us); zgemm 512 x 640 x 2000 takes 148 us N T, 155 us T T (tested: 148 and
+    // 158 us; a plain loop that checks a ragged range throughout: 145 and 151 us).
+    // More register sets of loads in flight measured no faster (two for the 64 x 64
+    // complex tile, three for the 64 x 64 real one: n = 1024 inverse 714 us either
+    // way, zpotrf + zpotri n = 8192 44.6 ms).
+    for (int k1 = 0; k1 < ntiles; k1++)
 #pragma unroll
-     for (int u = 0; u < NSET; u++) {
-      const int kt = kb + u;
-      if (NSET > 1 && kt >= ntiles) break;
-      if (kt + NSET < ntiles) {
+     for (int u = 0; u < 1; u++) {
+      const int kt = k1 + u;
+      if (kt + 1 < ntiles) {
         pa += a_kstride;
         pb += b_kstride;
-        load((kt + NSET) * KT, pa, pb, ra[u], rb[u]);
+        load((kt + 1) * KT, pa, pb);
       }
       const R *cA = sA + (kt & 1) * BUFA, *cB = sB + (kt & 1) * BUFB;
 #pragma unroll
@@ -472,7 +468,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) gemm_kernel(KParams<T> p) {
       }
       // The other buffer was last read in the previous step, which every
       // thread finished before the previous barrier.
-      if (kt + 1 < ntiles) store((kt + 1) & 1, ra[(u + 1) % NSET], rb[(u + 1) % NSET]);
+      if (kt + 1 < ntiles) store((kt + 1) & 1);
       __syncthreads();
     }
   } else {
