@@ -404,36 +404,49 @@ hipError_t trtri_device(hipStream_t s, char uplo, char diag, long n, T *A, long 
 }
 
 // Triangular square, lower L^H L, upper U U^H (the reference's loop is
-// lapack/dlauum.c:188-281).  Double and double complex up to order kSquareMax:
-// one product over the tiles of the result's triangle, with K cut to the rows
-// below both tiles, into the workspace, and a copy of the triangle.  Above, and
-// for single precision: [L11^H L11 + L21^H L21, .; L22^H L21, L22^H L22]
-// recursively (upper mirrors it), which keeps the workspace at a quarter of the
-// matrix.  Recursing down to the diagonal blocks is three launches per pair of
-// them; single precision keeps it because its diagonal blocks are squared in
-// double (leaves: beforehand, in one launch, since the products above a block
-// still read its factor; block b at leaves + b IB^2).
+// lapack/dlauum.c:188-281).  Double and double complex up to the order of a
+// leaf: one product over the tiles of the result's triangle, with K cut to the
+// rows below both tiles, into the workspace, and a copy of the triangle.  Above,
+// and for single precision: [L11^H L11 + L21^H L21, .; L22^H L21, L22^H L22]
+// recursively (upper mirrors it), which needs a quarter of the matrix as
+// workspace.  A leaf is of order kSquareMax (the workspace is then the whole
+// matrix, at most 512 MB, 1 GB complex), or half of the order where that much
+// memory is not free: dlauum n = 6001 2.0 ms, halved 2.4 ms, n = 8192 4.1 and
+// 5.6 ms.  Single precision recurses down to the diagonal blocks (three launches
+// per pair of them), which it squares in double (leaves: beforehand, in one
+// launch, since the products above a block still read its factor; block b at
+// leaves + b IB^2).
 constexpr long kSquareMax = 8192;
 
 template <typename T> constexpr bool is_single() { return std::is_same<T, float>::value || std::is_same<T, hc::zf>::value; }
 
+// order of the first half
 template <typename T>
-size_t lauum_rec_elems(long n) {
+long lauum_half(long n) {
   constexpr int IB = hc::diag_max<T>();
-  const long leaf = is_single<T>() ? IB : kSquareMax;
-  if (n <= leaf) return is_single<T>() ? 0 : (size_t)n * (size_t)n;
-  const long n1 = (n / 2 + IB - 1) / IB * IB;
-  return std::max({(size_t)n1 * (size_t)(n - n1), lauum_rec_elems<T>(n1), lauum_rec_elems<T>(n - n1)});
+  return (n / 2 + IB - 1) / IB * IB;
 }
 template <typename T>
-size_t lauum_ws_elems(long n) {
+long lauum_leaf(long n, bool halved) {
+  if (is_single<T>()) return hc::diag_max<T>();
+  return halved ? std::min(kSquareMax, lauum_half<T>(n)) : kSquareMax;
+}
+template <typename T>
+size_t lauum_rec_elems(long n, long leaf) {
+  if (n <= leaf) return is_single<T>() ? 0 : (size_t)n * (size_t)n;
+  const long n1 = lauum_half<T>(n);
+  return std::max({(size_t)n1 * (size_t)(n - n1), lauum_rec_elems<T>(n1, leaf), lauum_rec_elems<T>(n - n1, leaf)});
+}
+template <typename T>
+size_t lauum_ws_elems(long n, long leaf) {
   constexpr int IB = hc::diag_max<T>();
   const size_t leaves = is_single<T>() && n > IB ? (size_t)((n + IB - 1) / IB) * IB * IB : 0;
-  return lauum_rec_elems<T>(n) + leaves;
+  return lauum_rec_elems<T>(n, leaf) + leaves;
 }
 
 template <typename T>
-hipError_t lauum_rec(hipStream_t s, char uplo, long n, T *A, long lda, T *X, const T *leaves, const int *abort_flag) {
+hipError_t lauum_rec(hipStream_t s, char uplo, long n, long leaf, T *A, long lda, T *X, const T *leaves,
+                     const int *abort_flag) {
   constexpr int IB = hc::diag_max<T>();
   const T one = hc::from_real<T>(1.0), zero = hc::from_real<T>(0.0);
   const bool lower = uplo == 'L';
@@ -441,7 +454,7 @@ hipError_t lauum_rec(hipStream_t s, char uplo, long n, T *A, long lda, T *X, con
   o.abort_flag = abort_flag;
   if (is_single<T>()) {
     if (n <= IB) return hc::tri_copy<T>(s, uplo, n, leaves, IB, A, lda, abort_flag);
-  } else if (n <= kSquareMax) {
+  } else if (n <= leaf) {
     o.tri_grid = true;
     o.real_diag = hc::is_complex<T>::value;
     o.tri_out = lower ? hc::TRI_LOWER : hc::TRI_UPPER;
@@ -451,9 +464,9 @@ hipError_t lauum_rec(hipStream_t s, char uplo, long n, T *A, long lda, T *X, con
                             A, lda, zero, nullptr, 0, X, n, o));
     return hc::tri_copy<T>(s, uplo, n, X, n, A, lda, abort_flag);
   }
-  const long n1 = (n / 2 + IB - 1) / IB * IB, n2 = n - n1;
+  const long n1 = lauum_half<T>(n), n2 = n - n1;
   T *A11 = A, *A22 = A + n1 * lda + n1;
-  HC_TRY(lauum_rec(s, uplo, n1, A11, lda, X, leaves, abort_flag));
+  HC_TRY(lauum_rec(s, uplo, n1, leaf, A11, lda, X, leaves, abort_flag));
   if (lower) {
     T *A21 = A + n1;
     HC_TRY(hc::herk<T>(s, 'L', 'C', n1, n2, 1.0, A21, lda, 1.0, A11, lda, abort_flag));
@@ -467,20 +480,20 @@ hipError_t lauum_rec(hipStream_t s, char uplo, long n, T *A, long lda, T *X, con
     HC_TRY(hc::gemm_tile<T>(s, hc::OP_N, conj_op<T>(), n1, n2, n2, one, A12, lda, A22, lda, zero, nullptr, 0, X, n1, o));
     HC_TRY(hc::copy2d<T>(s, n1, n2, X, n1, A12, lda, abort_flag));
   }
-  return lauum_rec(s, uplo, n2, A22, lda, X, leaves == nullptr ? nullptr : leaves + (n1 / IB) * (long)IB * IB,
+  return lauum_rec(s, uplo, n2, leaf, A22, lda, X, leaves == nullptr ? nullptr : leaves + (n1 / IB) * (long)IB * IB,
                    abort_flag);
 }
 
 template <typename T>
-hipError_t lauum_device(hipStream_t s, char uplo, long n, T *A, long lda, T *X, const int *abort_flag) {
+hipError_t lauum_device(hipStream_t s, char uplo, long n, long leaf, T *A, long lda, T *X, const int *abort_flag) {
   T *leaves = nullptr;
   if constexpr (is_single<T>()) {
     constexpr int IB = hc::diag_max<T>();
     if (n <= IB) return hc::diag_lauum<T>(s, uplo, (int)n, A, lda, abort_flag);
-    leaves = X + lauum_rec_elems<T>(n);
+    leaves = X + lauum_rec_elems<T>(n, leaf);
     HC_TRY(hc::diag_lauum_blocks<T>(s, uplo, n, IB, A, lda, leaves, abort_flag));
   }
-  return lauum_rec<T>(s, uplo, n, A, lda, X, leaves, abort_flag);
+  return lauum_rec<T>(s, uplo, n, leaf, A, lda, X, leaves, abort_flag);
 }
 
 // Copies the device info word back and waits for the handle's streams.
@@ -521,15 +534,26 @@ CUresult potrf_api(const char *name, CULAPACKhandle h, CBlasUplo uplo, size_t n,
 template <typename T>
 CUresult triangle_ops(CULAPACKhandle h, CBlasUplo uplo, CBlasDiag diag, size_t n, T *A, size_t lda, bool invert,
                       bool square, long *info) {
-  const size_t elems = std::max(invert ? trtri_ws_elems<T>((long)n) : 0, square ? lauum_ws_elems<T>((long)n) : 0);
+  long leaf = lauum_leaf<T>((long)n, false);
+  auto bytes = [&]() {
+    return std::max(invert ? trtri_ws_elems<T>((long)n) : 0, square ? lauum_ws_elems<T>((long)n, leaf) : 0) * sizeof(T) +
+           256;
+  };
   void *ws = nullptr;
-  HC_CHECK(workspace(h, elems * sizeof(T) + 256, &ws));
+  hipError_t e = workspace(h, bytes(), &ws);
+  if (e == hipErrorOutOfMemory && square) {  // a quarter of the matrix suffices
+    (void)hipGetLastError();
+    leaf = lauum_leaf<T>((long)n, true);
+    e = workspace(h, bytes(), &ws);
+  }
+  HC_CHECK(e);
   const bool scan = invert && diag == CBlasNonUnit;
   const int *flag = scan ? h->dinfo : nullptr;
   if (scan) HC_CHECK(hc::diag_zero_scan<T>(h->stream, (char)uplo, (long)n, A, (long)lda, h->dinfo));
   if (invert)
     HC_CHECK(trtri_device<T>(h->stream, (char)uplo, (char)diag, (long)n, A, (long)lda, static_cast<T *>(ws), flag));
-  if (square) HC_CHECK(lauum_device<T>(h->stream, (char)uplo, (long)n, A, (long)lda, static_cast<T *>(ws), flag));
+  if (square)
+    HC_CHECK(lauum_device<T>(h->stream, (char)uplo, (long)n, leaf, A, (long)lda, static_cast<T *>(ws), flag));
   if (scan) return finish(h, info);
   HC_CHECK(hipStreamSynchronize(h->stream));
   return CUDA_SUCCESS;
