@@ -137,3 +137,22 @@ def test_herk_ignores_imaginary_diagonal(gpu, blas, prec, uplo, n, k):
     torch.cuda.synchronize()
     assert torch.equal(factor_of(clean, n, uplo), factor_of(dirty, n, uplo))
     assert (factor_of(dirty, n, uplo).diagonal().imag == 0).all()
+
+
+@pytest.mark.parametrize("prec", "SD")
+@pytest.mark.parametrize("uplo", "LU")
+def test_potrf_long_panels(gpu, lapack, prec, uplo):
+    """Panels with at least 8192 rows left apply the factored slices to each
+    new one: the first two or three of this order."""
+    dtype, n = TYPES[prec], 9293
+    A = spd(n, n, dtype)
+    lda = n + 3
+    W = store(A, uplo, lda, dtype)
+    st, info = getattr(gpu, f"cu{prec}potrf")(lapack, ord(uplo), n, gpu.ptr(W), lda)
+    torch.cuda.synchronize()
+    assert st == 0 and info == 0
+    L = factor_of(W, n, uplo)
+    eps = np.finfo(np.float32 if prec == "S" else np.float64).eps
+    err = (torch.linalg.norm(A - L @ L.mT) / torch.linalg.norm(A)).item()
+    assert err <= 10 * n * eps, err
+    assert torch.isnan(W[:, n:]).all()

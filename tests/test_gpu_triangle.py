@@ -86,3 +86,38 @@ def test_potri_singular_is_untouched(gpu, lapack, prec, uplo):
     torch.cuda.synchronize()
     assert st == 0 and info == k + 1
     assert torch.equal(torch.nan_to_num(W), torch.nan_to_num(before))
+
+
+@pytest.mark.parametrize("uplo", "LU")
+def test_trtri_large_tiles(gpu, lapack, uplo):
+    """Levels that take the larger product tile, with a ragged last pair."""
+    n = 6001
+    M = triangle(n, n, torch.float64, uplo)
+    W = store(M, uplo, n + 1, torch.float64)
+    st, info = gpu.cuDtrtri(lapack, ord(uplo), gpu.NonUnit, n, gpu.ptr(W), n + 1)
+    torch.cuda.synchronize()
+    assert st == 0 and info == 0
+    X, L = factor_of(W, n, uplo), M if uplo == "L" else M.mH
+    cond = (torch.linalg.norm(L) * torch.linalg.norm(X)).item()
+    eye = torch.eye(n, device="cuda", dtype=torch.float64)
+    assert torch.linalg.norm(X @ L - eye).item() <= 10 * n * eps_of("D") * cond
+    assert torch.isnan(W[:, n:]).all()
+
+
+@pytest.mark.parametrize("uplo", "LU")
+def test_potri_halved_square(gpu, lapack, uplo):
+    """Above the order that is squared in one product: two halves and the
+    products between them."""
+    n = 8301
+    A = spd(n, n, torch.float64)
+    M = torch.linalg.cholesky(A)
+    W = store(M if uplo == "L" else M.mH, uplo, n + 1, torch.float64)
+    st, info = gpu.cuDpotri(lapack, ord(uplo), n, gpu.ptr(W), n + 1)
+    torch.cuda.synchronize()
+    assert st == 0 and info == 0
+    X = factor_of(W, n, uplo)
+    X = torch.tril(X) + torch.tril(X, -1).mT
+    eye = torch.eye(n, device="cuda", dtype=torch.float64)
+    err = (torch.linalg.norm(A @ X - eye) / (torch.linalg.norm(A) * torch.linalg.norm(X))).item()
+    assert err <= 10 * n * eps_of("D"), err
+    assert torch.isnan(W[:, n:]).all()
