@@ -148,13 +148,10 @@ CUresult cuPotrfBatchedPlanCreate(CULAPACKhandle h, CBlasUplo uplo, char precisi
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return nv[a] > nv[b]; });
   // persistent grids: every CU filled to the kernel's occupancy (a workgroup
-  // that waits for a slot would start its share late); the inverse kernels
-  // take fewer per CU when the autotuner measured that faster
-  // ($CUCHOLESKY_BATCHED_PER_CU caps both)
+  // that waits for a slot would start its share late; $CUCHOLESKY_BATCHED_PER_CU
+  // caps it)
   const char *env = std::getenv("CUCHOLESKY_BATCHED_PER_CU");
   const int forced = env != nullptr ? std::atoi(env) : 0;
-  const int tuned = hc::tuned_batched_per_cu(precision, true);
-  const int inv_cap = forced > 0 ? forced : (tuned > 0 ? tuned : 1 << 20);
   for (size_t i = 0; i < count; i++) p->reg_count[hc::batched_reg_class(nv[i])]++;
   const bool dbl = precision == 'D';
   for (int c = 0; c < 3; c++) {
@@ -163,7 +160,7 @@ CUresult cuPotrfBatchedPlanCreate(CULAPACKhandle h, CBlasUplo uplo, char precisi
     const int inv = dbl ? hc::potri_batched_reg_blocks_per_cu<double>((char)uplo, c)
                         : hc::potri_batched_reg_blocks_per_cu<float>((char)uplo, c);
     p->reg_grid[c] = cus * (forced > 0 ? std::min(forced, occ) : occ);
-    p->inv_grid[c] = cus * std::min(inv_cap, inv);
+    p->inv_grid[c] = cus * (forced > 0 ? std::min(forced, inv) : inv);
   }
   hipError_t e = hipMalloc(&p->d_cnt, 3 * sizeof(int));
   if (e == hipSuccess) e = hipMemcpy(p->d_cnt, p->reg_count, 3 * sizeof(int), hipMemcpyHostToDevice);

@@ -1,11 +1,9 @@
 // Block sizes chosen by measurement.
 //
 // cuda-cholesky_amd/autotune.py times the factorisations over a grid of
-// outer block sizes, and the persistent schedule of the batched
-// factorisation, on the GPU at hand and writes the winners to a text table,
-// one line per entry:
+// outer block sizes, tile choices and caps on the GPU at hand and writes the
+// winners to a text table, one line per entry:
 //     potrf_nb <precision> <n_max> <nb>
-//     batched_per_cu <precision> <inverse> <workgroups per CU>
 //     gemm_tile <family> <min_tiles>
 //     panel_launch <precision> <0|1>
 //     trailing_cap <precision> <t_max> <workgroups>
@@ -45,9 +43,6 @@ std::vector<Entry> &table() {
   static std::vector<Entry> t;
   return t;
 }
-
-// batched_per_cu entries, indexed [precision D/S][inverse]; 0 = none
-int g_batched_per_cu[2][2] = {{0, 0}, {0, 0}};
 
 // gemm_tile entries by family letter; 0 = none
 long g_tile_min[26] = {};
@@ -96,9 +91,6 @@ void load() {
       g_cap[prec[0] - 'A'][0] = n_max;
       g_cap[prec[0] - 'A'][1] = nb;
     }
-    else if (std::strcmp(key, "batched_per_cu") == 0 && (prec[0] == 'D' || prec[0] == 'S') &&
-             (n_max == 0 || n_max == 1) && nb > 0 && nb <= 64)
-      g_batched_per_cu[prec[0] == 'S' ? 1 : 0][n_max] = (int)nb;
   }
   std::fclose(f);
 }
@@ -112,11 +104,6 @@ long tuned_potrf_nb(char prec, long n) {
   for (const Entry &e : table())
     if (e.prec == prec && n <= e.n_max) return e.nb;
   return 0;
-}
-
-int tuned_batched_per_cu(char prec, bool inverse) {
-  std::call_once(g_once, load);
-  return g_batched_per_cu[prec == 'S' ? 1 : 0][inverse ? 1 : 0];
 }
 
 long tuned_tile_min(char family, long dflt) {
