@@ -7,6 +7,9 @@ entries do not show it.  The bars are 10 n eps times the norms of the factors of
 the residual, with no condition number: a row-by-row substitution meets them
 with two digits to spare.
 """
+from decimal import Decimal, localcontext
+from fractions import Fraction
+
 import numpy as np
 import pytest
 import torch
@@ -128,3 +131,52 @@ def test_batched_inverse_residual(gpu, lapack, uplo):
         X = torch.tril(X) + torch.tril(X, -1).mT
         err = norm(A @ X - torch.eye(n, device="cuda", dtype=X.dtype)) / (norm(A) * norm(X))
         assert err <= 10 * n * EPS, (n, err)
+
+
+def exact_logdet(M):
+    """Pivots in rational arithmetic, their logarithms with 50 digits."""
+    n = len(M)
+    F = [[Fraction(float(v)) for v in row] for row in M]
+    with localcontext() as ctx:
+        ctx.prec = 50
+        total = Decimal(0)
+        for k in range(n):
+            total += Decimal(F[k][k].numerator).ln() - Decimal(F[k][k].denominator).ln()
+            for i in range(k + 1, n):
+                f = F[i][k] / F[k][k]
+                for j in range(k, n):
+                    F[i][j] -= f * F[k][j]
+        return float(total)
+
+
+@pytest.mark.parametrize("n", [2, 3, 5])
+def test_small_logdet_is_exact_to_the_condition(gpu, lapack, n):
+    """Log-determinants of ill-conditioned small matrices from the batched plan
+    and from the task-graph plan against exact arithmetic.  L L^T = A + E with
+    ||E|| <= (n + 1) eps n ||A|| moves the log-determinant by at most sqrt(n)
+    ||E|| / s_min, the n logarithms and their sum by 10 n eps relative."""
+    count = 150
+    rng = np.random.default_rng(n)
+    G = rng.standard_normal((count, n, n))
+    A = G @ np.swapaxes(G, 1, 2) / n + np.exp(rng.uniform(np.log(1e-8), 0.0, count))[:, None, None] * np.eye(n)
+    A = np.tril(A) + np.swapaxes(np.tril(A, -1), 1, 2)
+    want = np.array([exact_logdet(M) for M in A])
+    bound = (n ** 1.5 * (n + 1) * np.linalg.cond(A) + 10 * n * np.maximum(1.0, np.abs(want))) * EPS
+    sizes, offs, offb = [n] * count, [i * n * n for i in range(count)], [i * n for i in range(count)]
+    W = torch.from_numpy(A.reshape(-1).copy()).cuda()
+    A0 = W.clone()
+    logdet = torch.zeros(2, count, device="cuda", dtype=torch.float64)
+    info = torch.zeros(count, device="cuda", dtype=torch.int32)
+    with gpu.BatchedPlan(lapack, gpu.Lower, "D", sizes, offs) as plan:
+        assert plan.run(gpu.ptr(W), gpu.ptr(logdet[0]), gpu.ptr(info), torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+    assert (info == 0).all()
+    B = torch.ones(count * n, device="cuda", dtype=torch.float64)
+    X, Ainv, iters = torch.zeros_like(B), torch.zeros_like(A0), torch.zeros_like(info)
+    with gpu.BatchedSolvePlan(lapack, gpu.Lower, sizes, offs, 1, offb) as plan:
+        assert plan.run(gpu.ptr(A0), gpu.ptr(B), gpu.ptr(X), gpu.ptr(Ainv), gpu.ptr(iters), gpu.ptr(logdet[1]),
+                        gpu.ptr(info)) == 0
+        torch.cuda.synchronize()
+    assert (info == 0).all()
+    for got in logdet.cpu().numpy():
+        assert np.all(np.abs(got - want) <= bound)
