@@ -219,11 +219,11 @@ constexpr int diag_lds_elems() {
 // the same SIMD, is worker 6, which has no row; the workers, at a lower issue
 // priority, keep up with it because a row in registers leaves one LDS operand
 // per product.  One CU takes about 10000 cycles to read the block from HBM
-// (longer than two leaves): leaf 0 overlaps the left half of every row, leaf 1
-// the right half.  One 128 x 128 double
-// block alone: 24.5 us between events (36 us with a column-by-column leaf in a
-// layout of its own, the tiles in LDS, the write-out in wave 0 and the block
-// loaded element by element).
+// (longer than two leaves): leaf 0 overlaps the left three quarters of the tile
+// columns, leaf 1 the rest.  One 128 x 128 double block alone: 24.5 us between
+// events, 19.8 us in a kernel trace (36 us between events with a column-by-column
+// leaf in a layout of its own, the tiles in LDS, the write-out in wave 0 and the
+// block loaded element by element).
 template <typename T, typename ST, int NMAX, bool ZEROS, typename Src>
 __device__ __forceinline__ int diag_block_factor(const Src &src, bool failed, T *S, int &flag, int lower, int n,
                                                  ST *A, long lda, ST *W, long ldw) {
@@ -315,7 +315,7 @@ __device__ __forceinline__ int diag_block_factor(const Src &src, bool failed, T 
   const int wk = wave == 4 ? NW - 2 : (wave < 4 ? wave - 1 : wave - 2);  // worker
   const int row = wk + 2 < np ? wk + 2 : -1;
   TileAcc<T> R[NPMAX];  // the worker's tile row
-  constexpr int HALF = NPMAX * 6 / 8;
+  constexpr int FIRST = NPMAX * 6 / 8;  // tile columns loaded beside leaf 0
   // its tiles LO .. HI - 1
   auto take = [&](auto lo, auto hi) __attribute__((always_inline)) {
     constexpr int LO = decltype(lo)::value, HI = decltype(hi)::value;
@@ -330,7 +330,7 @@ __device__ __forceinline__ int diag_block_factor(const Src &src, bool failed, T 
       }
     });
   };
-  take(std::integral_constant<int, 0>{}, std::integral_constant<int, HALF>{});
+  take(std::integral_constant<int, 0>{}, std::integral_constant<int, FIRST>{});
   if (failed) return -1;
   __syncthreads();
   TileAcc<T> sacc;  // S_{p+1,wk}, carried from phase B to the next phase A
@@ -354,7 +354,7 @@ __device__ __forceinline__ int diag_block_factor(const Src &src, bool failed, T 
   int bad = flag;  // of leaf p (padding never fails, so it is below n)
   if (bad >= 0) return bad;
   if (np > 1) __syncthreads();
-  take(std::integral_constant<int, HALF>{}, std::integral_constant<int, NPMAX>{});
+  take(std::integral_constant<int, FIRST>{}, std::integral_constant<int, NPMAX>{});
   for (int p = 0;; p++) {
     // phase B of step p
     if (wk >= p && row > 0) {  // A_IJ -= L_Ip L_Jp^H, I = row
@@ -836,7 +836,9 @@ panel_potrf_kernel(int m, int jb, ST *A, long lda, ST *ws, int *flags, int epoch
 // element 5e-14, this 4e-14, without the correction 1e-12, joining inverted
 // halves (X21 = -X22 L21 X11) 3e-13 (and 7e-11 in L X - I at nugget 1e-10).
 // Waves w and w + 4 share a SIMD and take columns w and 7 - w, so that every
-// matrix core has the same products.
+// matrix core has the same products.  40 blocks of 128 x 128 doubles in a launch:
+// 20 us (108 us as a substitution by columns in registers, one barrier per
+// column).
 // ---------------------------------------------------------------------------
 template <int NMAX>
 constexpr int tri_lds_elems() {

@@ -4,7 +4,7 @@
 // Every step runs on the GPU.  The reference copies each diagonal block to the
 // host, factors it there and copies it back (lapack/dpotrf.c:263-275); here a
 // single-workgroup LDS kernel factors the block and also returns its inverse,
-// so the panel solve becomes a matrix-core GEMM and the loop never waits for
+// so the panel solve becomes a matrix-core product and the loop never waits for
 // the host.  `info` lives in device memory; kernels issued after a failed
 // pivot see it and do nothing, and one copy at the end returns it.
 #include "api_util.h"
@@ -67,9 +67,9 @@ template <typename T> char prec_of(bool bf16) {
 }
 
 // Panel factorisation of columns [j, j + jb) (lower; rows [j, j + jb) for
-// upper), all rows below, in IB-column slices: diagonal block (LDS kernel,
-// factor + inverse), panel solve as a GEMM with the inverse, and the rest of
-// the panel updated with the slice.
+// upper), all rows below, in IB-column slices: diagonal block (factor +
+// inverse in one workgroup), panel solve with the inverse, and the rest of the
+// panel updated with the slice (or each slice with all before it).
 template <typename T>
 hipError_t factor_panel(CULAPACKhandle h, hipStream_t s, bool lower, long n, T *A, long lda, T *W,
                         long j, long jb) {
@@ -229,8 +229,8 @@ hipError_t potrf_device(CULAPACKhandle h, char uplo, long n, T *A, long lda, T *
   // panel is slower beside the trailing update: its resident workgroups keep
   // the CUs the 16-bit update's workgroups need (one per CU, all of the LDS
   // and registers), and its left-looking steps put two 128^3 products on one
-  // CU on the critical path (dpotrf n = 16384 34.5 ms against 33.5 ms; FP16
-  // solve n = 32768 59.8 ms against 57.6 ms).
+  // CU on the critical path (dpotrf n = 16384 37.7 ms against 29.1 ms, 32.7 ms
+  // with NB = 512; FP16 solve n = 32768 56.0 ms against 48.6 ms).
   const bool one_launch = lower && !hc::is_complex<T>::value && NB <= hc::kPanelMaxCols &&
                           hc::tuned_panel_launch(prec_of<T>(bf16), false);
   if (one_launch) HC_TRY(panel_resources(h));
