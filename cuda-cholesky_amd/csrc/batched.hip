@@ -397,20 +397,22 @@ potrf_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
 //     X_JJ, with the tiles of L read from the matrix as operand fragments: no
 //     exchange between waves.  k runs as 4 lk + s there, so that in lower
 //     storage a lane's four elements are one load, and so are its four of X;
-//   * the rows replace L in the matrix, the waves read their columns of X back,
-//     and form their columns of the result, R_ij = sum_{K>=i} X_Ki^T X_Kj,
-//     i ascending, with X_Ki from the matrix; R_ij takes the registers of X_ij,
-//     which no later i needs;
-//   * R replaces X in the matrix.
+//   * the rows go to LDS, or for n > 128, where the triangle does not fit it,
+//     replace L in the matrix; the waves read their columns of X back and form
+//     their columns of the result, R_ij = sum_{K>=i} X_Ki^T X_Kj, i ascending,
+//     with X_Ki from there too; R_ij takes the registers of X_ij, which no later
+//     i needs;
+//   * R replaces L or X in the matrix.
 // X by rows has a small X L - I, which is what A X^T X - I needs.  By columns
 // (X_IJ = -X_II sum L_IK X_KJ, small L X - I) the columns would stay where they
 // are, but the residual of the inverse on graded factors is 30 to 500 times
 // larger: squared-exponential covariances, nugget 1e-8, ||A R - I|| / (||A||
 // ||R||) 3e-15 by rows, 2e-12 by columns at n = 128.
-// Factor and inverse of 20000 matrices, n in [8, 256]: FP32 storage 6.6 ms
-// (upper 6.7), of which the factor 2.4 (2.6), FP64 8.0 ms (8.3); by columns 7.5
+// Factor and inverse of 20000 matrices, n in [8, 256]: FP32 storage 6.4 ms
+// (upper 6.6), of which the factor 2.4 (2.6), FP64 7.9 ms (8.2); by columns 7.5
 // (7.0) and 7.8 ms (9.2); a 4-wave workgroup that streams every tile of a matrix
-// through memory at every step 9.8 (8.4) and 11.1 ms (10.8).  The fully
+// through memory at every step 9.8 (8.4) and 11.1 ms (10.8).  10000 matrices, n in
+// [65, 128], FP64: X in LDS 2.45 ms, through the matrix 2.94 ms.  The fully
 // unrolled tile products are more code than the instruction cache holds, but
 // rolled loops over K spilled 200 to 800 registers (rows and columns are indexed
 // at compile time).
@@ -422,9 +424,12 @@ potri_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
   constexpr int NWI = NPMAX / 2;
   const int count = cnt[CLS];
   order += CLS == 2 ? 0 : (CLS == 1 ? cnt[2] : cnt[2] + cnt[1]);
+  constexpr bool XL = CLS < 2;             // X below the diagonal tiles in LDS
   __shared__ double D[NPMAX * LEAF * LL];  // X_II
+  __shared__ double XB[XL ? NPMAX * (NPMAX - 1) / 2 * LEAF * LL : 1];
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto xtile = [&](int I, int J) { return XB + (I * (I - 1) / 2 + J) * LEAF * LL; };  // I > J
   for (int t = blockIdx.x; t < count; t += gridDim.x) {
     const int idx = __builtin_amdgcn_readfirstlane(order[t]);
     const int n = __builtin_amdgcn_readfirstlane(nvec[idx]);
@@ -459,11 +464,17 @@ potri_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
         l[s] = ok ? x : 0.0;
       }
     };
-    // a tile of X that is whole (all but a ragged last tile row) and that lies
-    // along columns in memory is kept transposed there, so that the loads of
+    // in the matrix, a tile of X that is whole (all but a ragged last tile row) and
+    // that lies along columns in memory is kept transposed, so that the loads of
     // X_Ki^T below run along memory; X_JJ stays in LDS
     auto transposed = [&](int I) { return LOWER && (I + 1) * LEAF <= n; };
     auto load_x = [&](int K, int J, auto &l) __attribute__((always_inline)) {
+      if constexpr (XL) {
+        const double *p = xtile(K, J) + li * LL + lk;
+#pragma unroll
+        for (int s = 0; s < 4; s++) l[s] = p[4 * s];
+        return;
+      }
       if (transposed(K)) {
         const ST *p = tile_at(K, J);
 #pragma unroll
@@ -532,7 +543,7 @@ potri_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
         Z[at(d)] = acc;
       });
     });
-    __syncthreads();  // every read of L is done
+    if (!XL) __syncthreads();  // every read of L is done
     rows([&](auto Sec, int I) __attribute__((always_inline)) {
       constexpr int sec = decltype(Sec)::value, TM = sec ? NPMAX / 2 : NPMAX;
       t16::static_for<1, TM>([&](auto Dc) {
@@ -540,6 +551,11 @@ potri_batched_reg_kernel(const int *cnt, const int *nvec, const long *offs, cons
         if (d > I) return;
         const int J = I - d;
         const v4d &z = Z[sec ? NPMAX - d : d];
+        if constexpr (XL) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) xtile(I, J)[(4 * lk + r) * LL + li] = z[r];
+          return;
+        }
         // X(li, 4 lk + r): along memory in upper storage, and in lower storage where the tile is transposed
         if ((I + 1) * LEAF <= n) {
           const row4 x = {(ST)z[0], (ST)z[1], (ST)z[2], (ST)z[3]};
